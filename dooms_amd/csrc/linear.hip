@@ -399,10 +399,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(LinearParams p) {
     // row's last 8 columns instead, finite values that meet the zero padding
     const int kp = (p.K + kTK - 1) / kTK * kTK;
     const int kc = threadIdx.x % 8;  // the same for every j: 256 is a multiple of 8
-    const half_t * a0 = p.xh + (int64_t)min(m0 + (int)threadIdx.x / 8, p.M - 1) * kp + 8 * kc;
-    const half_t * b0 = w + (int64_t)min(n0 + (int)threadIdx.x / 8, p.N - 1) * p.K;
-    const int64_t a_step = (int64_t)(kThreads / 8) * kp, b_step = (int64_t)(kThreads / 8) * p.K;  // 32 rows per j
-    const int brow_max = p.N - 1 - n0, arow_max = p.M - 1 - m0;  // rows past N (M) repeat the last row
+    int64_t a_off[kChunks], b_off[kChunks];  // this thread's rows of the tiles, 32 apart
+#pragma unroll
+    for (int j = 0; j < kChunks; j++) {
+        a_off[j] = (int64_t)gemm_load_row(m0, (int)threadIdx.x / 8 + 32 * j, p.M) * kp + 8 * kc;
+        b_off[j] = (int64_t)gemm_load_row(n0, (int)threadIdx.x / 8 + 32 * j, p.N) * p.K;
+    }
     // two register sets: step i's tiles travel in set i % 2, loaded two steps before they are stored into LDS
     u32x4 ar[2][kChunks], br[2][kChunks];
     auto load = [&](int step, auto S) __attribute__((always_inline)) {
@@ -411,10 +413,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_kernel(LinearParams p) {
         const int bcol = min(k0 + 8 * kc, p.K - 8);
 #pragma unroll
         for (int j = 0; j < kChunks; j++) {
-            const int64_t aoff = (int)threadIdx.x / 8 + 32 * j <= arow_max ? j * a_step : (int64_t)(arow_max - (int)threadIdx.x / 8) * kp;
-            ar[st][j] = load16(a0 + aoff + k0);
-            const int64_t boff = (int)threadIdx.x / 8 + 32 * j <= brow_max ? j * b_step : (int64_t)(brow_max - (int)threadIdx.x / 8) * p.K;
-            br[st][j] = load16(b0 + boff + bcol);
+            ar[st][j] = load16(p.xh + a_off[j] + k0);
+            br[st][j] = load16(w + b_off[j] + bcol);
         }
     };
     auto store = [&](int buf, auto S) __attribute__((always_inline)) {

@@ -193,6 +193,12 @@ constexpr int kLinearMaxMats = 64;
 constexpr int kLinearGemvMaxRows = 8;        // M up to this runs the f32-input GEMV, above it the MFMA GEMM
 constexpr size_t kLinearGemvLds = 64 * 1024;  // staged input rows up to this many bytes per workgroup
 
+// The row that load `row` of a GEMM tile starting at row `first` reads, of `rows` in all: rows past the last repeat it
+// (finite values that are multiplied and never stored), so that no load leaves the operand.
+__host__ __device__ inline int32_t gemm_load_row(int32_t first, int32_t row, int32_t rows) {
+    return first + row < rows - 1 ? first + row : rows - 1;
+}
+
 struct LinearParams {
     const float * x;
     const float * gamma;

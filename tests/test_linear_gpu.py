@@ -128,6 +128,12 @@ def test_gemm_step_counts(device, M, N, K):
     run(device, 20 + K, M, N, K, norm=True, bias=True)
 
 
+@pytest.mark.parametrize("M,N", [(9, 8), (12, 200), (16, 16), (17, 12)])
+def test_gemm_few_rows(device, M, N):
+    """Fewer rows or columns than a tile's loads cover: every load past them repeats the last one."""
+    run(device, 60 + M, M, N, 128, bias=True, accumulate=True)
+
+
 def test_gemm_big_tiles_ragged(device):
     """A product with enough 256 x 256 tiles for the large-tile GEMM: M and N not multiples of 256 (rows and
     columns past them repeat the last one and are never stored), 5 steps of 32 columns, with the RMS normalization,
