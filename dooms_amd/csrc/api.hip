@@ -752,6 +752,10 @@ int32_t linear_params(const mx_linear_desc * desc, int32_t count, const uint16_t
     p.x = X;
     p.gamma = gamma;
     p.xh = static_cast<mx::half_t *>(workspace);
+    p.plan = mx::LinearPlan{-1, 1, 0, 0};
+    if (need) p.plan = mx::linear_plan(d.M, d.N, d.K, count, ws_bytes - need);
+    p.counters = reinterpret_cast<uint32_t *>(static_cast<char *>(workspace) + need);
+    p.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + need + mx::linear_counter_bytes(p.plan));
     p.x_stride = d.x_stride;
     p.y_stride = d.y_stride;
     p.M = d.M;
@@ -1039,7 +1043,9 @@ MX_ATTN_API size_t mx_linear_workspace_bytes(const mx_linear_desc * desc) {
         fail(MX_ATTN_INVALID_ARGUMENT, "desc is null");
         return 0;
     }
-    return linear_ws_bytes(*desc);
+    const size_t rows = linear_ws_bytes(*desc);
+    if (!rows || desc->N < 1 || desc->K < 1) return rows;
+    return rows + mx::linear_plan(desc->M, desc->N, desc->K, 1, SIZE_MAX).bytes;
 }
 
 MX_ATTN_API int32_t mx_linear(const mx_linear_desc * desc, int32_t count, const uint16_t * const * W, const float * X,

@@ -65,20 +65,6 @@ __device__ __forceinline__ void collect2(const float * p, float & a, float & b) 
     b = __uint_as_float((uint32_t)(v >> 32));
 }
 
-// 16-byte device-scope (sc1) buffer loads: coherent across the XCDs, a quarter of the instructions of 4-byte atomic
-// loads. The resource is built from a wave-uniform base (a per-lane base would make the compiler loop over the distinct
-// descriptors of the wave); lanes differ in their byte offsets.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t dev_rsrc(const void * base) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0x7fffffff, 0x00020000);
-}
-constexpr int kCpolSc1 = 16;  // the cache-policy bit that makes a buffer access device-scope on gfx950
-__device__ __forceinline__ u32x4 load16_dev(__amdgpu_buffer_rsrc_t r, int byte_off) {
-    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, byte_off, 0, kCpolSc1));
-}
-__device__ __forceinline__ void store16_dev(__amdgpu_buffer_rsrc_t r, int byte_off, float4_t v) {
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, byte_off, 0, kCpolSc1);
-}
-
 // XCD-local publishing (the XCD-mapped grid, where every split of a tile runs on one XCD): plain stores, complete once
 // they reach that XCD's L2, where the merging workgroup's device-scope loads find them (a store-load round trip on one
 // XCD: 0.96 us, against 1.50 us with device-scope stores). Batch 1 at 8192 keys 11.07-11.35 -> 10.70-10.89 us per

@@ -16,11 +16,10 @@
 //     (8 with eight input rows) of 2 or 4 loads in flight per lane. The input rows' loads go out first, in one
 //     batch, then the first sweeps of weight loads, so that the staging waits only for the input; the dot products
 //     stay f32 and are reduced across the wave at the end.
-//   * M > 8 (prompt): stage_kernel writes each input row once as half(x * gamma * scale) into the workspace (the
-//     reference stages the same values per tile); gemm_kernel, v_mfma_f32_32x32x16_f16 on 128 x 128 output tiles, K in
-//     steps of 64 through LDS (double buffer, rows padded to 72 halves so that the 16-byte operand reads of 16
-//     consecutive rows hit 16 distinct 4-bank groups), the step after next loading while the current step multiplies.
-//     Each wave owns a 64 x 64 block (2 x 2 MFMA tiles); two workgroups per CU.
+//   * M > 8 (prompt, batched decode): stage_kernel writes each input row once as half(x * gamma * scale) into the
+//     workspace (the reference stages the same values per tile). Products with enough tiles for every CU run on
+//     gemm_big_tile, 256-row tiles of 8 waves; the others on gemm_split_tile, smaller tiles and K cut into parts, so
+//     that a product of few rows streams its weights through the whole chip. linear_plan picks by a fitted cost.
 //   * Several matrices with the same input and shape (the cross cache's K and V of every layer) run in one launch.
 //   * mx_linear runs these kernels only: no vendor GEMM library is loaded or linked.
 
@@ -45,6 +44,8 @@ constexpr int kWaves = kThreads / kWave;
 template <bool NORM>
 __global__ __launch_bounds__(kThreads) void stage_kernel(LinearParams p) {
     __shared__ float red[kWaves];
+    if (p.plan.splits > 1)  // the split GEMM's counters (one per thread of the whole grid; the grid has rows > 8)
+        for (int i = blockIdx.x * kThreads + threadIdx.x; i < p.plan.tiles; i += gridDim.x * kThreads) p.counters[i * kCounterStride] = 0u;
     const float * row = p.x + (int64_t)blockIdx.x * p.x_stride;
     const int kp = (p.K + 63) / 64 * 64;  // staged rows are zero-padded to a multiple of 64 columns
     half_t * dst = p.xh + (int64_t)blockIdx.x * kp;
@@ -376,136 +377,24 @@ __global__ __launch_bounds__(kGemvMaxWaves * kWave) void gemv_kernel(LinearParam
     }
 }
 
-// ---- M > 8: MFMA GEMM on the staged half rows, 128 x 128 tiles, K in steps of 64 ----
-constexpr int kTM = 128, kTN = 128, kTK = 64;
-constexpr int kPitch = kTK + 8;  // halves per staged row: the 16-byte reads of 16 consecutive rows hit distinct banks
-constexpr int kChunks = kTM * (kTK / 8) / kThreads;  // 16-byte chunks per thread per tile and step (4)
-
-template <bool OUT16>
-__global__ __launch_bounds__(kThreads, 2) void gemm_kernel(LinearParams p) {
-    __shared__ half_t xs[2][kTM * kPitch];
-    __shared__ half_t ws[2][kTN * kPitch];
-    const int n_tiles = (p.N + kTN - 1) / kTN, m_tiles = (p.M + kTM - 1) / kTM;
-    // consecutive work items share a weight tile (different token tiles); contiguous ranges per XCD
-    const uint32_t t = xcd_remap(blockIdx.x, (uint32_t)(p.count * n_tiles * m_tiles));
-    const int mt = t % m_tiles, nt = (t / m_tiles) % n_tiles, mi = t / (m_tiles * n_tiles);
-    const int m0 = mt * kTM, n0 = nt * kTN;
-    const half_t * w = p.w[mi];
-    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int l32 = lane % 32, hi = lane / 32;
-
-    // staging map: chunk c = threadIdx.x + 256 j is row c / 8, columns 8 (c % 8) .. + 8 of the step. The staged rows are
-    // zero-padded to a multiple of 64 columns (kp); a weight column past K (K an odd multiple of 32) is read from the
-    // row's last 8 columns instead, finite values that meet the zero padding
-    const int kp = (p.K + kTK - 1) / kTK * kTK;
-    const int kc = threadIdx.x % 8;  // the same for every j: 256 is a multiple of 8
-    int64_t a_off[kChunks], b_off[kChunks];  // this thread's rows of the tiles, 32 apart
-#pragma unroll
-    for (int j = 0; j < kChunks; j++) {
-        a_off[j] = (int64_t)gemm_load_row(m0, (int)threadIdx.x / 8 + 32 * j, p.M) * kp + 8 * kc;
-        b_off[j] = (int64_t)gemm_load_row(n0, (int)threadIdx.x / 8 + 32 * j, p.N) * p.K;
-    }
-    // two register sets: step i's tiles travel in set i % 2, loaded two steps before they are stored into LDS
-    u32x4 ar[2][kChunks], br[2][kChunks];
-    auto load = [&](int step, auto S) __attribute__((always_inline)) {
-        constexpr int st = decltype(S)::value;
-        const int k0 = step * kTK;
-        const int bcol = min(k0 + 8 * kc, p.K - 8);
-#pragma unroll
-        for (int j = 0; j < kChunks; j++) {
-            ar[st][j] = load16(p.xh + a_off[j] + k0);
-            br[st][j] = load16(w + b_off[j] + bcol);
-        }
-    };
-    auto store = [&](int buf, auto S) __attribute__((always_inline)) {
-        constexpr int st = decltype(S)::value;
-#pragma unroll
-        for (int j = 0; j < kChunks; j++) {
-            const int c = threadIdx.x + kThreads * j, row = c / 8, kc = c % 8;
-            *reinterpret_cast<u32x4 *>(&xs[buf][row * kPitch + 8 * kc]) = ar[st][j];
-            *reinterpret_cast<u32x4 *>(&ws[buf][row * kPitch + 8 * kc]) = br[st][j];
-        }
-    };
-
-    float16_t acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
-
-    const int wm = wave / 2, wn = wave % 2;  // this wave's 64 x 64 block
-    const int a_base = (64 * wm + l32) * kPitch + 8 * hi;
-    const int b_base = (64 * wn + l32) * kPitch + 8 * hi;
-    const int nk = kp / kTK;
-    using S0 = std::integral_constant<int, 0>;
-    using S1 = std::integral_constant<int, 1>;
-    load(0, S0{});
-    store(0, S0{});
-    load(min(1, nk - 1), S1{});
-    load(min(2, nk - 1), S0{});
-    // step ib: its tiles are in LDS buffer ib % 2; step ib + 1's go from register set (ib + 1) % 2 into the other
-    // buffer, and that set is refilled with step ib + 3's
-    // The loads and stores are unconditional (past the last step the last step's tiles are loaded again and go into a
-    // buffer nobody reads), so the loop has one path and the waits for one register set leave the other set in flight.
-    auto step = [&](int ib, auto S) __attribute__((always_inline)) {
-        const int buf = ib & 1;
-        __syncthreads();  // step ib is in buffer buf; buffer buf ^ 1 is free
-        store(buf ^ 1, S);
-        load(min(ib + 3, nk - 1), S);
-        const half_t * a_s = xs[buf];
-        const half_t * b_s = ws[buf];
-#pragma unroll
-        for (int ks = 0; ks < kTK / 16; ks++) {
-            half8_t a[2], b[2];
-#pragma unroll
-            for (int i = 0; i < 2; i++) a[i] = as_half8(*reinterpret_cast<const u32x4 *>(a_s + a_base + 32 * i * kPitch + 16 * ks));
-#pragma unroll
-            for (int j = 0; j < 2; j++) b[j] = as_half8(*reinterpret_cast<const u32x4 *>(b_s + b_base + 32 * j * kPitch + 16 * ks));
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = mfma32x32x16(a[i], b[j], acc[i][j]);
-        }
-    };
-    int ib = 0;
-    for (; ib + 1 < nk; ib += 2) {
-        step(ib, S1{});
-        step(ib + 1, S0{});
-    }
-    if (ib < nk) step(ib, S1{});
-
-    // lane holds Y[m0 + 64 wm + 32 i + 8 (v / 4) + 4 hi + v % 4][n0 + 64 wn + 32 j + l32]
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int n = n0 + 64 * wn + 32 * j + l32;
-            if (n < p.N) store_col16<OUT16>(p, mi, n, m0 + 64 * wm + 32 * i + 4 * hi, acc[i][j]);
-        }
-}
-
-// ---- M > 8, large products: 256 x 256 tiles of 8 waves (each 128 x 64, 4 x 2 MFMA tiles), K in steps of 32 ----
+// ---- M > 8, large products: 256 x 256 tiles of 8 waves (each 128 x 64, 4 x 2 MFMA tiles), K in steps of 64 ----
 // A 128 x 128 tile streams 64 bytes per clock and CU from L2 at the MFMA rate, the whole of an XCD's L2 bandwidth;
 // 256 x 256 halves the bytes per product (and 128 x 64 per wave cuts the LDS reads per product by a quarter). The
 // tiles go from HBM/L2 straight into LDS (global_load_lds_dwordx4: lane l's 16 bytes land at byte 16 l of the
-// instruction's 1 KB destination), three buffers deep (the loads of step s + 2 in flight while step s multiplies), no
-// registers in between. An operand tile (256 rows x 32 columns, 64 bytes per row) is 16 blocks of 16 rows, one load
-// instruction each; 16-byte chunk c of row r sits at 16 (c ^ ((r % 16) / 4)) within its row's 64 bytes, so the 16-byte
-// operand reads of 16 consecutive rows at one chunk land on 16 distinct 4-bank groups. 96 KB of LDS: one workgroup per
-// CU, two waves per SIMD.
-// BN = 128 (256 x 128 tiles, 8 waves of 64 x 64) and BN = 192 (256 x 192, 8 waves of 64 x 96) serve products whose
-// 256 x 256 tiles would leave CUs idle.
+// instruction's 1 KB destination), two buffers (the loads of step s + 1 in flight while step s multiplies), no
+// registers in between. An operand tile (256 rows x 64 columns) is two column groups of 16 blocks of 16 rows x 64
+// bytes, one load instruction each; 16-byte chunk c of row r sits at 16 (c ^ ((r % 16) / 4)) within its row's 64 bytes,
+// so the 16-byte operand reads of 16 consecutive rows at one chunk land on 16 distinct 4-bank groups. 128 KB of LDS:
+// one workgroup per CU, two waves per SIMD.
+// BN = 192 (256 x 192, 8 waves of 64 x 96) serves products whose 256 x 256 tiles would leave CUs idle.
 constexpr int kBM = 256;
 constexpr int kGemmCUs = 256;
 constexpr int kBigWaves = 8, kBigThreads = kBigWaves * kWave;
-// WC: columns per wave (64, or 96 for 256 x 192 tiles: 8 waves of 64 x 96). BK: columns per step, 32 (three buffers)
-// or 64 (two buffers, half the barriers and load instructions per product; K a multiple of 64).
-template <bool OUT16, int BN, int WC = 64, int BK = 32>
+// WC: columns per wave (64, or 96 for 256 x 192 tiles: 8 waves of 64 x 96).
+template <bool OUT16, int BN, int WC>
 __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
-    constexpr int kBN = BN, kBK = BK;
-    constexpr int kBigBufs = BK == 32 ? 3 : 2;
+    constexpr int kBN = BN, kBK = 64;
+    constexpr int kBigBufs = 2;
     constexpr int kBigLoads = kBM * kBK * 2 / 1024 / kBigWaves;  // 1 KB direct loads of A per wave and step
     constexpr int RA = kBM / 16, RBB = BN / 16;                  // 16-row blocks per chunk group of A and of B
     constexpr int WN = BN / WC, WM = kBigWaves / WN;         // waves along N and along M
@@ -580,10 +469,9 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
         if (a < nk) issue(a, a);
     for (int s = 0; s < nk; s++) {
         const int buf = s % kBigBufs;
-        // this wave's loads of step s are complete (those of up to kBigBufs - 2 later steps may be in flight), then
-        // every wave's are; the buffer refilled below was last read in step s - 1
-        if (kBigBufs > 2 && s + 1 < nk) __builtin_amdgcn_s_waitcnt(0x0F70 | (kBigLoads + BLoads));  // vmcnt(next step)
-        else __builtin_amdgcn_s_waitcnt(0x0F70);                                                     // vmcnt(0)
+        // this wave's loads of step s are complete, then every wave's are; the buffer refilled below was last read in
+        // step s - 1
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -592,92 +480,39 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
         // wait for those), all of the step's in flight, the products of each 16-column slice behind their reads
         const uint32_t xa = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) half_t *)xs[buf] + 2 * 32 * (kBM / WM) * wm;
         const uint32_t wa = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) half_t *)ws[buf] + 2 * 32 * WC * wn;
-        if constexpr (BK == 64) {
-            // 4 slices of 16 columns: slices s + 1's reads in flight behind slice s's products (at most 2 slices of
-            // reads outstanding, within the 15 that lgkmcnt counts); the waits are ordered by sched_barrier
-            constexpr int R = kBigMI + kBigNJ;  // reads per slice
-            u32x4 fa[4][kBigMI], fb[4][kBigNJ];
-            auto reads = [&](auto KS) __attribute__((always_inline)) {
-                constexpr int ks = decltype(KS)::value;
-                const uint32_t ra_ = xa + 2 * (rd[ks % 2] + 512 * RA * (ks / 2)), rb_ = wa + 2 * (rd[ks % 2] + 512 * RBB * (ks / 2));
-                static_for<0, kBigMI>([&](auto I) __attribute__((always_inline)) {
-                    u32x4 r;
-                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(ra_), "i"(2 * 1024 * decltype(I)::value));
-                    fa[ks][decltype(I)::value] = r;
-                });
-                static_for<0, kBigNJ>([&](auto J) __attribute__((always_inline)) {
-                    u32x4 r;
-                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(rb_), "i"(2 * 1024 * decltype(J)::value));
-                    fb[ks][decltype(J)::value] = r;
-                });
-            };
-            reads(std::integral_constant<int, 0>{});
-            reads(std::integral_constant<int, 1>{});
-            static_for<0, 4>([&](auto KS) __attribute__((always_inline)) {
-                constexpr int ks = decltype(KS)::value;
-                if constexpr (ks < 3) asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(R) : "memory");
-                else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int i = 0; i < kBigMI; i++)
-#pragma unroll
-                    for (int j = 0; j < kBigNJ; j++)
-                        acc[i][j] = mfma32x32x16(as_half8(fa[ks][i]), as_half8(fb[ks][j]), acc[i][j]);
-                __builtin_amdgcn_sched_barrier(0);
-                if constexpr (ks + 2 < 4) reads(std::integral_constant<int, ks + 2>{});
+        // 4 slices of 16 columns: slices s + 1's reads in flight behind slice s's products (at most 2 slices of
+        // reads outstanding, within the 15 that lgkmcnt counts); the waits are ordered by sched_barrier
+        constexpr int R = kBigMI + kBigNJ;  // reads per slice
+        u32x4 fa[4][kBigMI], fb[4][kBigNJ];
+        auto reads = [&](auto KS) __attribute__((always_inline)) {
+            constexpr int ks = decltype(KS)::value;
+            const uint32_t ra_ = xa + 2 * (rd[ks % 2] + 512 * RA * (ks / 2)), rb_ = wa + 2 * (rd[ks % 2] + 512 * RBB * (ks / 2));
+            static_for<0, kBigMI>([&](auto I) __attribute__((always_inline)) {
+                u32x4 r;
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(ra_), "i"(2 * 1024 * decltype(I)::value));
+                fa[ks][decltype(I)::value] = r;
             });
-        } else {
-            u32x4 fa[2][kBigMI], fb[2][kBigNJ];
-            static_for<0, 2>([&](auto KS) __attribute__((always_inline)) {
-                constexpr int ks = decltype(KS)::value;
-                const uint32_t ra_ = xa + 2 * rd[ks], rb_ = wa + 2 * rd[ks];
-                static_for<0, kBigMI>([&](auto I) __attribute__((always_inline)) {
-                    constexpr int i = decltype(I)::value;
-                    u32x4 r;
-                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(ra_), "i"(2 * 1024 * i));
-                    fa[ks][i] = r;
-                });
-                static_for<0, kBigNJ>([&](auto J) __attribute__((always_inline)) {
-                    constexpr int j = decltype(J)::value;
-                    u32x4 r;
-                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(rb_), "i"(2 * 1024 * j));
-                    fb[ks][j] = r;
-                });
+            static_for<0, kBigNJ>([&](auto J) __attribute__((always_inline)) {
+                u32x4 r;
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(rb_), "i"(2 * 1024 * decltype(J)::value));
+                fb[ks][decltype(J)::value] = r;
             });
-            static_for<0, 2>([&](auto KS) __attribute__((always_inline)) {
-                constexpr int ks = decltype(KS)::value;
-                // slice 0 waits for its reads (slice 1's in flight), slice 1 for all: one wait per slice, tied to the
-                // slice's fragments
-                static_assert((kBigNJ == 2 && (kBigMI == 4 || kBigMI == 2)) || (kBigNJ == 3 && kBigMI == 2),
-                              "the waits below name every fragment");
-                if constexpr (kBigNJ == 3) {
-                    if constexpr (ks == 0)
-                        asm volatile("s_waitcnt lgkmcnt(5)" : "+v"(fa[0][0]), "+v"(fa[0][1]), "+v"(fb[0][0]), "+v"(fb[0][1]),
-                                     "+v"(fb[0][2]));
-                    else
-                        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[1][0]), "+v"(fa[1][1]), "+v"(fb[1][0]), "+v"(fb[1][1]),
-                                     "+v"(fb[1][2]));
-                } else if constexpr (kBigMI == 4) {
-                    if constexpr (ks == 0)
-                        asm volatile("s_waitcnt lgkmcnt(6)" : "+v"(fa[0][0]), "+v"(fa[0][1]), "+v"(fa[0][2]), "+v"(fa[0][3]),
-                                     "+v"(fb[0][0]), "+v"(fb[0][1]));
-                    else
-                        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[1][0]), "+v"(fa[1][1]), "+v"(fa[1][2]), "+v"(fa[1][3]),
-                                     "+v"(fb[1][0]), "+v"(fb[1][1]));
-                } else {
-                    if constexpr (ks == 0)
-                        asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(fa[0][0]), "+v"(fa[0][1]), "+v"(fb[0][0]), "+v"(fb[0][1]));
-                    else
-                        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[1][0]), "+v"(fa[1][1]), "+v"(fb[1][0]), "+v"(fb[1][1]));
-                }
+        };
+        reads(std::integral_constant<int, 0>{});
+        reads(std::integral_constant<int, 1>{});
+        static_for<0, 4>([&](auto KS) __attribute__((always_inline)) {
+            constexpr int ks = decltype(KS)::value;
+            if constexpr (ks < 3) asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(R) : "memory");
+            else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int i = 0; i < kBigMI; i++)
+            for (int i = 0; i < kBigMI; i++)
 #pragma unroll
-                    for (int j = 0; j < kBigNJ; j++)
-                        acc[i][j] = mfma32x32x16(as_half8(fa[ks][i]), as_half8(fb[ks][j]), acc[i][j]);
-                __builtin_amdgcn_sched_barrier(0);
-            });
-        }
+                for (int j = 0; j < kBigNJ; j++)
+                    acc[i][j] = mfma32x32x16(as_half8(fa[ks][i]), as_half8(fb[ks][j]), acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (ks + 2 < 4) reads(std::integral_constant<int, ks + 2>{});
+        });
     }
 
     // lane holds Y[m0 + (256 / WM) wm + 32 i + 8 (v / 4) + 4 hi + v % 4][n0 + WC wn + 32 j + l32]
@@ -690,13 +525,277 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
         }
 }
 
-// K in steps of 64 columns when K is a multiple of 64 (BK = 64), else 32
-template <bool OUT16, int BK>
-__global__ __launch_bounds__(kBigThreads, 1) void gemm_big_kernel(LinearParams p) { gemm_big_tile<OUT16, 256, 64, BK>(p); }
-template <bool OUT16, int BK>
-__global__ __launch_bounds__(kBigThreads, 1) void gemm_mid_kernel(LinearParams p) { gemm_big_tile<OUT16, 128, 64, BK>(p); }
-template <bool OUT16, int BK>
-__global__ __launch_bounds__(kBigThreads, 1) void gemm_w192_kernel(LinearParams p) { gemm_big_tile<OUT16, 192, 96, BK>(p); }
+template <bool OUT16>
+__global__ __launch_bounds__(kBigThreads, 1) void gemm_big_kernel(LinearParams p) { gemm_big_tile<OUT16, 256, 64>(p); }
+template <bool OUT16>
+__global__ __launch_bounds__(kBigThreads, 1) void gemm_w192_kernel(LinearParams p) { gemm_big_tile<OUT16, 192, 96>(p); }
+
+// ---- M > 8, products with too few 256-row tiles for the chip: BM x BN tiles of 4 waves, K cut into p.plan.splits parts ----
+// Few rows are bound by the weights' stream from HBM (24 x 4096 x 4096: 33.5 MB, 5.2 us at 6.4 TB/s), which needs every
+// CU loading: with whole K a product of N = 4096 has 32 column tiles for 256 CUs, so the parts of K make up the rest
+// (4 parts of 64-column tiles: 256 workgroups). Each workgroup keeps NBUF - 1 steps of both operands in flight straight
+// into LDS (48 to 96 KB), in whole row slices of 256 (BK = 128) or 128 bytes, so its few steps arrive about together. Row r of a
+// tile lies whole in LDS with its 16-byte chunks permuted by the row (chunk ^ r % 16, or ^ r / 2 % 8 with 128-byte rows): the
+// 16-byte operand reads of 16 rows at one chunk hit 16 distinct 4-bank groups. The weights are MFMA operand A, so that
+// a lane holds 4 consecutive outputs of one row (16-byte stores).
+template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF>
+__device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
+    constexpr int WN = kWaves / WM;                        // waves along the weight rows
+    constexpr int MI = BM / WM / 16, NJ = BN / WN / 16;    // 16 x 16 MFMA tiles per wave
+    constexpr int CH = BK / 8, RPB = 64 / CH;              // 16-byte chunks per row, rows per 1 KB load block
+    constexpr int XB = BM / RPB, WB = BN / RPB;            // load blocks of a step
+    constexpr int LPS = (XB + WB) / kWaves;                // loads per wave and step
+    constexpr int KS = BK / 32;                            // MFMA steps per K step
+    static_assert((XB + WB) % kWaves == 0 && MI >= 1 && NJ >= 1 && LPS * (NBUF - 1) < 64, "whole loads and tiles");
+    __shared__ __attribute__((aligned(1024))) half_t sm[NBUF][(BM + BN) * BK];
+    __shared__ int s_last;
+    const int n_tiles = (p.N + BN - 1) / BN, m_tiles = (p.M + BM - 1) / BM, S = p.plan.splits;
+    uint32_t t = xcd_remap(blockIdx.x, (uint32_t)(p.plan.tiles * S));
+    const int mt = t % m_tiles;
+    t /= m_tiles;
+    const int split = t % S;
+    t /= S;
+    const int nt = t % n_tiles, mi = t / n_tiles;
+    const int tile = (mi * n_tiles + nt) * m_tiles + mt;
+    const int m0 = mt * BM, n0 = nt * BN;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const int kp = (p.K + 63) / 64 * 64;
+    const int steps = BK == 64 ? kp / 64 : p.K / BK, s0 = (int)((int64_t)split * steps / S), nk = (int)((int64_t)(split + 1) * steps / S) - s0;
+
+    // load block j = i kWaves + wave of a step: RPB rows x BK columns; lane l fills position l % CH of row l / CH with
+    // chunk (l % CH) ^ swizzle(row)
+    auto swz = [](int row) { return BK == 128 ? row & 15 : (row >> 1) & 7; };
+    const char * const xg = reinterpret_cast<const char *>(p.xh + (int64_t)m0 * kp);
+    const char * const wg = reinterpret_cast<const char *>(p.w[mi] + (int64_t)n0 * p.K);
+    uint32_t off[LPS];
+#pragma unroll
+    for (int i = 0; i < LPS; i++) {
+        const int j = i * kWaves + wave;
+        const bool isx = j < XB;
+        const int row = (isx ? j : j - XB) * RPB + lane / CH;
+        const int r = isx ? gemm_load_row(m0, row, p.M) - m0 : gemm_load_row(n0, row, p.N) - n0;
+        off[i] = (uint32_t)r * (uint32_t)(isx ? kp : p.K) * 2 + 16 * ((lane % CH) ^ swz(row));
+    }
+    auto issue = [&](int step, int buf) __attribute__((always_inline)) {
+        const int64_t k0 = (int64_t)(s0 + step) * BK * 2;
+        // the last step of a K that is an odd multiple of 32: the staged rows are zero-padded, the weights' chunks past
+        // the row read the four before them (finite values that meet the zeros)
+        const bool half_step = BK == 64 && (s0 + step) * BK + BK > p.K;
+#pragma unroll
+        for (int i = 0; i < LPS; i++) {
+            const int j = i * kWaves + wave;
+            const char * src = (j < XB ? xg : wg) + k0;
+            uint32_t o = off[i];
+            if (BK == 64 && __builtin_expect(half_step, 0) && j >= XB && ((lane % CH) ^ swz((j - XB) * RPB + lane / CH)) >= 4) o -= 64;
+            __builtin_amdgcn_global_load_lds(src + o, (__attribute__((address_space(3))) void *)&sm[buf][512 * j], 16, 0, 0);
+        }
+    };
+    float4_t acc[MI][NJ];
+#pragma unroll
+    for (int i = 0; i < MI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    const int wm = wave / WN, wn = wave % WN, l16 = lane % 16, grp = lane / 16;
+    uint32_t rd[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) rd[ks] = (uint32_t)l16 * BK * 2 + 16 * ((4 * ks + grp) ^ swz(l16));
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) half_t *)sm[0];
+#pragma unroll
+    for (int a = 0; a < NBUF - 1; a++)
+        if (a < nk) issue(a, a);
+    for (int s = 0; s < nk; s++) {
+        const int buf = s % NBUF;
+        const int later = min(NBUF - 2, nk - 1 - s);
+        static_for<0, NBUF - 1>([&](auto R) __attribute__((always_inline)) {
+            constexpr int n = decltype(R)::value * LPS;
+            if (later == decltype(R)::value) __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
+        });
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (s + NBUF - 1 < nk) issue(s + NBUF - 1, (s + NBUF - 1) % NBUF);
+        const uint32_t xa = lds0 + (uint32_t)buf * (BM + BN) * BK * 2 + wm * (BM / WM) * BK * 2;
+        const uint32_t wa = lds0 + (uint32_t)buf * (BM + BN) * BK * 2 + (BM + wn * (BN / WN)) * BK * 2;
+        u32x4 fx[KS][MI], fw[KS][NJ];
+        auto reads = [&](auto KSC) __attribute__((always_inline)) {
+            constexpr int ks = decltype(KSC)::value;
+            static_for<0, MI>([&](auto I) __attribute__((always_inline)) {
+                u32x4 r;
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(xa + rd[ks]), "i"(32 * BK * decltype(I)::value));
+                fx[ks][decltype(I)::value] = r;
+            });
+            static_for<0, NJ>([&](auto J) __attribute__((always_inline)) {
+                u32x4 r;
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(wa + rd[ks]), "i"(32 * BK * decltype(J)::value));
+                fw[ks][decltype(J)::value] = r;
+            });
+        };
+        reads(std::integral_constant<int, 0>{});
+        reads(std::integral_constant<int, 1>{});
+        static_for<0, KS>([&](auto KSC) __attribute__((always_inline)) {
+            constexpr int ks = decltype(KSC)::value;
+            if constexpr (ks + 1 < KS) asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(MI + NJ) : "memory");
+            else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) acc[i][j] = mfma16x16x32(as_half8(fw[ks][j]), as_half8(fx[ks][i]), acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (ks + 2 < KS) reads(std::integral_constant<int, ks + 2>{});
+        });
+    }
+
+    if (S > 1) {
+        // the partial tile out with device-scope stores, complete before the tile's counter counts it in; the part that
+        // completes the count sums every part in order (its own read back too: the result does not depend on which part
+        // came last) and writes the output
+        constexpr int64_t TF = (int64_t)BM * BN;  // floats per partial tile
+        const __amdgpu_buffer_rsrc_t prs = dev_rsrc(p.part + (int64_t)tile * S * TF);
+        const int fb = ((wave * MI * NJ) * kWave + lane) * 16;
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) store16_dev(prs, split * (int)TF * 4 + fb + (i * NJ + j) * kWave * 16, acc[i][j]);
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (threadIdx.x == 0)
+            s_last = __hip_atomic_fetch_add(p.counters + (int64_t)tile * kCounterStride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(S - 1);
+        __syncthreads();
+        if (!s_last) return;
+        __builtin_amdgcn_s_waitcnt(0);
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+        constexpr int SC = MI * NJ >= 16 ? 1 : 16 / (MI * NJ);  // parts in flight per round
+        for (int k0 = 0; k0 < S; k0 += SC) {
+            float4_t v[SC][MI][NJ];
+#pragma unroll
+            for (int e = 0; e < SC; e++)
+                if (k0 + e < S)
+#pragma unroll
+                    for (int i = 0; i < MI; i++)
+#pragma unroll
+                        for (int j = 0; j < NJ; j++)
+                            v[e][i][j] = __builtin_bit_cast(float4_t, load16_dev(prs, (k0 + e) * (int)TF * 4 + fb + (i * NJ + j) * kWave * 16));
+#pragma unroll
+            for (int e = 0; e < SC; e++)
+                if (k0 + e < S)
+#pragma unroll
+                    for (int i = 0; i < MI; i++)
+#pragma unroll
+                        for (int j = 0; j < NJ; j++) acc[i][j] += v[e][i][j];
+        }
+    }
+
+    // lane holds Y[m0 + wm BM / WM + 16 i + l16][n0 + wn BN / WN + 16 j + 4 grp + v]
+    const float * b = (p.flags & kLinearBias) ? p.bias[mi] : nullptr;
+    const bool accum = p.flags & kLinearAccumulate;
+    const int mb = m0 + wm * (BM / WM) + l16, nb = n0 + wn * (BN / WN) + 4 * grp;
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const int n = nb + 16 * j;
+        if (n >= p.N) continue;
+        const bool whole = n + 3 < p.N;
+        if (b) {
+            float bv[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++) bv[v] = b[min(n + v, p.N - 1)];
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[i][j][v] += bv[v];
+        }
+        if (accum) {
+            float prev[MI][4];
+#pragma unroll
+            for (int i = 0; i < MI; i++) {
+                const int64_t o = (int64_t)min(mb + 16 * i, p.M - 1) * p.y_stride + n;
+#pragma unroll
+                for (int v = 0; v < 4; v++) prev[i][v] = 0.f;
+                if (whole) {
+                    if constexpr (OUT16) {
+                        const half4_t h = *reinterpret_cast<const half4_t *>(static_cast<const half_t *>(p.y[mi]) + o);
+#pragma unroll
+                        for (int v = 0; v < 4; v++) prev[i][v] = (float)h[v];
+                    } else {
+                        const float4_t h = *reinterpret_cast<const float4_t *>(static_cast<const float *>(p.y[mi]) + o);
+#pragma unroll
+                        for (int v = 0; v < 4; v++) prev[i][v] = h[v];
+                    }
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; v++)
+                        if (n + v < p.N) prev[i][v] = OUT16 ? (float)static_cast<const half_t *>(p.y[mi])[o + v] : static_cast<const float *>(p.y[mi])[o + v];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[i][j][v] += prev[i][v];
+        }
+#pragma unroll
+        for (int i = 0; i < MI; i++) {
+            const int m = mb + 16 * i;
+            if (m >= p.M) continue;
+            const int64_t o = (int64_t)m * p.y_stride + n;
+            if constexpr (OUT16) {
+                half_t * y = static_cast<half_t *>(p.y[mi]) + o;
+                if (whole) *reinterpret_cast<half4_t *>(y) = half4_t{(half_t)acc[i][j][0], (half_t)acc[i][j][1], (half_t)acc[i][j][2], (half_t)acc[i][j][3]};
+                else
+#pragma unroll
+                    for (int v = 0; v < 3; v++)
+                        if (n + v < p.N) y[v] = (half_t)acc[i][j][v];
+            } else {
+                float * y = static_cast<float *>(p.y[mi]) + o;
+                if (whole) *reinterpret_cast<float4_t *>(y) = acc[i][j];
+                else
+#pragma unroll
+                    for (int v = 0; v < 3; v++)
+                        if (n + v < p.N) y[v] = acc[i][j][v];
+            }
+        }
+    }
+}
+
+template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF>
+__global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(LinearParams p) { gemm_split_tile<OUT16, BM, BN, WM, BK, NBUF>(p); }
+
+// The GEMM's tile shapes and what a product costs on each, in microseconds, fitted (least relative squares, 8 % rms) to
+// 4700 measured launches: 9 to 4096 rows of the decoders' projections, every shape with 1 to 12 parts of K.
+//   t = 4.5 + 0.2 M K / 1e6 (staging) + 1.06 M N / 1e6 (output)                       the same for every shape
+//     + rounds * (tile + steps * step)     steps of 64 columns per part; a round is one workgroup per CU, or two where
+//                                          per_cu is 2 (a part round of at most one per CU takes step1, else step2)
+//     + (parts > 1) * (merge * (1 + parts * tile bytes / 64 KB) + part_mb * partial MB)
+// Picking the cheapest is within 1.1 % of the measured best on average over those products (the worst 19 %). What the
+// split buys, against the 128 x 128 tiles with whole K that took every product of few tiles (us, staging included):
+// 24 x 4096 x 4096 47.9 -> 12.9, 64 x 4096 x 4096 49.0 -> 15.3, 256 x 4096 x 4096 51.0 -> 24.6, 24 x 4096 x 14336
+// 147 -> 29.4, 512 x 1152 x 896 19.1 -> 10.0, 1024 x 3584 x 3584 50.2 -> 46.
+struct GemmCfg {
+    int bm, bn, bk, threads, per_cu;
+    float step1, step2, tile, merge, part_mb;
+    void (*k32)(LinearParams);
+    void (*k16)(LinearParams);
+};
+constexpr int kGemmCfgs = 8;
+constexpr int kMaxParts = 12, kMaxSplitGrid = 1024;  // the fitted range
+const GemmCfg & gemm_cfg(int c) {
+#define MX_SPLIT(BM, BN, WM, BK, NB, CU, ...) \
+    {BM, BN, BK, kThreads, CU, __VA_ARGS__, gemm_split_kernel<false, BM, BN, WM, BK, NB>, gemm_split_kernel<true, BM, BN, WM, BK, NB>}
+    static const GemmCfg cfgs[kGemmCfgs] = {
+        MX_SPLIT(16, 64, 1, 128, 6, 1, 0.219f, 0.f, 0.315f, 0.539f, 1.588f),
+        MX_SPLIT(32, 64, 1, 128, 3, 2, 0.250f, 0.402f, 0.f, 0.899f, 0.522f),
+        MX_SPLIT(64, 64, 2, 64, 4, 2, 0.340f, 0.553f, 0.f, 0.920f, 0.415f),
+        MX_SPLIT(128, 64, 2, 128, 3, 1, 0.421f, 0.f, 1.094f, 0.765f, 0.348f),
+        MX_SPLIT(128, 128, 2, 64, 4, 1, 0.640f, 0.f, 2.207f, 0.930f, 0.203f),
+        MX_SPLIT(128, 128, 2, 64, 2, 2, 0.887f, 1.078f, 0.f, 1.092f, 0.306f),
+        {256, 192, 64, kBigThreads, 1, 1.279f, 0.f, 8.563f, 0.f, 0.f, gemm_w192_kernel<false>, gemm_w192_kernel<true>},
+        {256, 256, 64, kBigThreads, 1, 1.609f, 0.f, 10.664f, 0.f, 0.f, gemm_big_kernel<false>, gemm_big_kernel<true>},
+    };
+#undef MX_SPLIT
+    return cfgs[c];
+}
 
 // Waves per workgroup: the (matrix, RW-row group) items spread evenly over the CUs, one workgroup per CU (the weight
 // stream of each CU then ends at the same time), up to 8 waves; beyond 2048 items, several workgroups of 8 per CU.
@@ -753,40 +852,40 @@ hipError_t launch_linear(const LinearParams & p, hipStream_t stream) {
     return launch_gemm(p, stream);
 }
 
-hipError_t launch_gemm(const LinearParams & p, hipStream_t stream) {
-    // 256-row tiles 256, 192 or 128 columns wide (one workgroup per CU), whichever costs the fewest rounds on the CUs
-    // times its width, the narrower tiles weighted for their lower efficiency (measured: the Llama-3-8B q|k|v chunk,
-    // 2048 x 6144, as 256 tiles of 256 x 192 rather than 192 of 256 x 256); when even the 256 x 128 tiles leave a
-    // quarter of the CUs idle, 128 x 128 tiles (three workgroups per CU)
-    const int mtl = (p.M + kBM - 1) / kBM;
-    const int64_t t256 = (int64_t)p.count * ((p.N + 255) / 256) * mtl, t192 = (int64_t)p.count * ((p.N + 191) / 192) * mtl,
-                  t128 = (int64_t)p.count * ((p.N + 127) / 128) * mtl;
-    const bool f16 = p.flags & kLinearOutF16;
-    if (4 * t128 >= 3 * kGemmCUs || 4 * t256 >= 3 * kGemmCUs) {
-        auto rounds = [](int64_t t) { return (double)((t + kGemmCUs - 1) / kGemmCUs); };
-        const double c256 = rounds(t256) * 256 * (4 * t256 >= 3 * kGemmCUs ? 1.0 : 1.35);  // a partial round idles CUs
-        const double c192 = rounds(t192) * 192 * 1.05 * (4 * t192 >= 3 * kGemmCUs ? 1.0 : 1.35);
-        const double c128 = rounds(t128) * 128 * 1.15;
-        const bool k64 = p.K % 64 == 0;
-        const int sel = 2 * (k64 ? 1 : 0) + (f16 ? 1 : 0);
-        void (*const big[4])(LinearParams) = {gemm_big_kernel<false, 32>, gemm_big_kernel<true, 32>,
-                                              gemm_big_kernel<false, 64>, gemm_big_kernel<true, 64>};
-        void (*const w192[4])(LinearParams) = {gemm_w192_kernel<false, 32>, gemm_w192_kernel<true, 32>,
-                                               gemm_w192_kernel<false, 64>, gemm_w192_kernel<true, 64>};
-        void (*const mid[4])(LinearParams) = {gemm_mid_kernel<false, 32>, gemm_mid_kernel<true, 32>,
-                                              gemm_mid_kernel<false, 64>, gemm_mid_kernel<true, 64>};
-        if (c256 <= c192 && c256 <= c128)
-            hipLaunchKernelGGL(big[sel], dim3((uint32_t)t256), dim3(kBigThreads), 0, stream, p);
-        else if (c192 <= c128)
-            hipLaunchKernelGGL(w192[sel], dim3((uint32_t)t192), dim3(kBigThreads), 0, stream, p);
-        else
-            hipLaunchKernelGGL(mid[sel], dim3((uint32_t)t128), dim3(kBigThreads), 0, stream, p);
-        return hipGetLastError();
+LinearPlan linear_plan(int32_t M, int32_t N, int32_t K, int32_t count, size_t avail) {
+    LinearPlan best{-1, 1, 0, 0};
+    float best_t = 0.f;
+    for (int i = 0; i < kGemmCfgs; i++) {
+        const GemmCfg & c = gemm_cfg(i);
+        // the split GEMM's 64-column shapes take any K (a multiple of 32), so that some shape always applies
+        if (K % (c.bk == 128 ? 128 : c.bm == kBM ? 64 : 32)) continue;
+        const int64_t tiles = (int64_t)count * ((N + c.bn - 1) / c.bn) * ((M + c.bm - 1) / c.bm);
+        const int ksteps = (K + c.bk - 1) / c.bk;
+        const int most = c.merge > 0.f ? (int)std::min<int64_t>(std::min(kMaxParts, ksteps), kMaxSplitGrid / tiles) : 1;
+        for (int s = 1; s <= std::max(most, 1); s++) {
+            const LinearPlan l{i, s, (int32_t)tiles, 0};
+            const size_t part_bytes = s > 1 ? (size_t)tiles * s * c.bm * c.bn * 4 : 0;
+            const size_t bytes = part_bytes + linear_counter_bytes(l);
+            if (bytes > avail) break;
+            const int64_t wgs = tiles * s, slots = (int64_t)kGemmCUs * c.per_cu, full = wgs / slots, rem = wgs % slots;
+            const float steps = (float)((ksteps + s - 1) / s) * (float)(c.bk / 64);
+            const float n1 = (float)((c.per_cu == 1 ? full : 0) + (rem > 0 && rem <= kGemmCUs ? 1 : 0));
+            const float n2 = (float)((c.per_cu == 1 ? 0 : full) + (rem > kGemmCUs ? 1 : 0));
+            float t = (n1 + n2) * c.tile + steps * (n1 * c.step1 + n2 * c.step2);
+            if (s > 1) t += c.merge * (1.f + (float)(s * c.bm * c.bn * 4) / 65536.f) + c.part_mb * (float)part_bytes * 1e-6f;
+            if (best.cfg < 0 || t < best_t) {
+                best = l;
+                best.bytes = bytes;
+                best_t = t;
+            }
+        }
     }
-    const int tiles = p.count * ((p.N + kTN - 1) / kTN) * ((p.M + kTM - 1) / kTM);
-    const dim3 grid((uint32_t)tiles);
-    if (p.flags & kLinearOutF16) hipLaunchKernelGGL(gemm_kernel<true>, grid, dim3(kThreads), 0, stream, p);
-    else hipLaunchKernelGGL(gemm_kernel<false>, grid, dim3(kThreads), 0, stream, p);
+    return best;
+}
+
+hipError_t launch_gemm(const LinearParams & p, hipStream_t stream) {
+    const GemmCfg & c = gemm_cfg(p.plan.cfg);
+    hipLaunchKernelGGL((p.flags & kLinearOutF16) ? c.k16 : c.k32, dim3((uint32_t)(p.plan.tiles * p.plan.splits)), dim3(c.threads), 0, stream, p);
     return hipGetLastError();
 }
 

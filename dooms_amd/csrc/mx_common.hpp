@@ -122,6 +122,20 @@ __device__ __forceinline__ half8_t as_half8(u32x4 v) { return __builtin_bit_cast
 // also counts against the LDS/scalar wait counter and so turns the waits for LDS into waits for memory.
 __device__ __forceinline__ u32x4 load16(const void * p) { return *(const __attribute__((address_space(1))) u32x4 *)(p); }
 
+// 16-byte device-scope (sc1) buffer loads: coherent across the XCDs, a quarter of the instructions of 4-byte atomic
+// loads. The resource is built from a wave-uniform base (a per-lane base would make the compiler loop over the distinct
+// descriptors of the wave); lanes differ in their byte offsets.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dev_rsrc(const void * base) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, 0x7fffffff, 0x00020000);
+}
+constexpr int kCpolSc1 = 16;  // the cache-policy bit that makes a buffer access device-scope on gfx950
+__device__ __forceinline__ u32x4 load16_dev(__amdgpu_buffer_rsrc_t r, int byte_off) {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, byte_off, 0, kCpolSc1));
+}
+__device__ __forceinline__ void store16_dev(__amdgpu_buffer_rsrc_t r, int byte_off, float4_t v) {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, byte_off, 0, kCpolSc1);
+}
+
 // Maps a workgroup index to a work index so that each XCD (the chip has 8, and consecutive workgroups are dealt out to
 // them round-robin) runs a contiguous range of the work order: neighbours in that order share keys/values in one L2.
 __device__ __forceinline__ uint32_t xcd_remap(uint32_t bid, uint32_t n) {

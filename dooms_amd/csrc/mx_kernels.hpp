@@ -199,10 +199,23 @@ __host__ __device__ inline int32_t gemm_load_row(int32_t first, int32_t row, int
     return first + row < rows - 1 ? first + row : rows - 1;
 }
 
+// How a product of more than kLinearGemvMaxRows rows runs.
+struct LinearPlan {
+    int32_t cfg;     // the GEMM's tile shape
+    int32_t splits;  // parts of K per tile
+    int32_t tiles;
+    size_t bytes;    // workspace behind the staged rows (counters, then partial tiles); 0 with one part
+};
+
 struct LinearParams {
     const float * x;
     const float * gamma;
     half_t * xh;    // [M][K] the staged input rows (M > 8): written by stage_kernel, read by the GEMM
+    // the split GEMM's (plan.splits > 1): partial tiles and one counter per tile, in the workspace behind the staged
+    // rows; stage_kernel zeroes the counters ahead of every GEMM
+    float * part;
+    uint32_t * counters;
+    LinearPlan plan;
     int64_t x_stride, y_stride;
     int32_t M, N, K, count;
     uint32_t flags;
@@ -219,6 +232,10 @@ hipError_t launch_fill_zero(void * p, size_t bytes, hipStream_t stream);
 // query rows one prefill workgroup covers (forced: a plan fixed by the caller, or 0)
 int prefill_rows_per_workgroup(int n_q, int n_head, int n_kv, int head_dim, int forced);
 hipError_t launch_prefill(const PrefillParams & p, int head_dim, hipStream_t stream);
+// counters of a split GEMM, each on a 256-byte line of its own
+inline size_t linear_counter_bytes(const LinearPlan & l) { return l.splits > 1 ? (size_t)l.tiles * kCounterStride * 4 : 0; }
+// avail: workspace bytes behind the staged rows that the plan may use
+LinearPlan linear_plan(int32_t M, int32_t N, int32_t K, int32_t count, size_t avail);
 hipError_t launch_linear(const LinearParams & p, hipStream_t stream);
 hipError_t launch_stage(const LinearParams & p, hipStream_t stream);  // M > 8: the staged half input rows
 hipError_t launch_gemm(const LinearParams & p, hipStream_t stream);   // M > 8: gemm_kernel on the staged rows

@@ -51,9 +51,12 @@ typedef struct mx_linear_desc {
 } mx_linear_desc;
 
 /*
- * Bytes of device workspace mx_linear needs for this descriptor: for M > 8, M * round_up(K, 64) halves (256-byte
- * rounded) for the input rows staged once as half(x * gamma * rms_scale) (the values the reference's matmul stages
- * per tile, with its rms_scale buffer folded in); 0 for M <= 8.
+ * Bytes of device workspace mx_linear asks for with this descriptor and one matrix; 0 for M <= 8. For M > 8:
+ * M * round_up(K, 64) halves (256-byte rounded) for the input rows staged once as half(x * gamma * rms_scale) (the
+ * values the reference's matmul stages per tile, with its rms_scale buffer folded in), and behind them, for products of
+ * too few tiles to fill the chip, the partial tiles of a K cut into parts. The staged rows are what a call must have;
+ * with less room behind them than asked for here it takes fewer parts (results agree within the summation order).
+ * Nothing needs to be initialized, and nothing is kept between calls.
  */
 MX_ATTN_API size_t mx_linear_workspace_bytes(const mx_linear_desc * desc);
 

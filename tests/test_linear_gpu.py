@@ -134,6 +134,44 @@ def test_gemm_few_rows(device, M, N):
     run(device, 60 + M, M, N, 128, bias=True, accumulate=True)
 
 
+@pytest.mark.parametrize("M", [9, 16, 17, 32, 33, 64, 65, 128, 129, 300])
+@pytest.mark.parametrize("N,K,opts", [
+    (136, 2048, dict(bias=True, accumulate=True)),         # K a multiple of 128: every tile shape, K in parts
+    (1029, 1152, dict(norm=True, y_pad=3)),                # the last columns of a row not a whole 16 bytes
+    (72, 1056, dict(accumulate=True, out_f16=True)),       # K an odd multiple of 32: the last step half padding
+    (200, 640, dict(bias=True, out_f16=True, count=3)),
+])
+def test_gemm_parts_of_k(device, M, N, K, opts):
+    """Few tiles: K is cut into parts merged by the last of a tile's workgroups; rows at the edges of every tile height,
+    columns that end inside a tile, and outputs written whole and in pieces."""
+    run(device, 80 + M + K, M, N, K, **opts)
+
+
+@pytest.mark.parametrize("M,N,K", [(24, 256, 4096), (200, 320, 1280)])
+def test_gemm_workspace_of_the_staged_rows_alone(device, M, N, K):
+    """A workspace with room for the staged rows only (and for a part of what the plan would take) still runs, with
+    fewer parts of K; calls in a row on one workspace left in any state agree bit for bit."""
+    rng = np.random.default_rng(M)
+    x = torch.from_numpy(rng.standard_normal((M, K), dtype=np.float32)).to(device)
+    w = torch.from_numpy((rng.standard_normal((N, K), dtype=np.float32) / np.sqrt(K)).astype(np.float16)).to(device)
+    ref = (x.half().double() @ w.double().T).cpu().numpy()
+    from dooms_amd import _lib
+    d = _lib.MxLinearDesc(M=M, N=N, K=K, flags=0, x_stride=K, y_stride=N, eps=1e-5, reserved=0)
+    staged, need = M * K * 2, _lib.linear_workspace_bytes(d)
+    assert need > staged  # these products are split
+    for nbytes in (staged, (staged + need) // 2, need):
+        ws = torch.full((nbytes,), 0xAB, dtype=torch.uint8, device=device)
+        outs = []
+        for _ in range(2):
+            y = torch.full((M, N), 7.0, device=device)
+            _lib.check(_lib.linear_raw(d, [w.data_ptr()], x.data_ptr(), [y.data_ptr()], 0, None, ws.data_ptr(), nbytes,
+                                       torch.cuda.current_stream().cuda_stream))
+            outs.append(y.cpu().numpy())
+        S = np.abs(x.half().double().cpu().numpy()) @ np.abs(w.double().cpu().numpy()).T
+        assert (np.abs(outs[0] - ref) <= 1e-5 * S + 1e-6).all()
+        assert np.array_equal(outs[0], outs[1])
+
+
 def test_gemm_big_tiles_ragged(device):
     """A product with enough 256 x 256 tiles for the large-tile GEMM: M and N not multiples of 256 (rows and
     columns past them repeat the last one and are never stored), 5 steps of 32 columns, with the RMS normalization,
