@@ -1,9 +1,12 @@
 """torch-tensor front end of the C ABI (plumbing: torch only supplies device memory and the stream).
 
 Every call goes through libmx_attn.so; there is no CPU or PyTorch fallback. Tensors must be CUDA (HIP) float16 with a
-unit stride along the feature dimension; row strides are taken from the tensors.
+unit stride along the feature dimension; row strides are taken from the tensors. The plain case of each entry point
+(tensors as documented, no tuning, a decode workspace of the caller's) runs in dooms_amd._native; everything else, and every
+refused argument, here.
 """
 import contextlib
+import ctypes
 import math
 
 import torch
@@ -32,6 +35,30 @@ def _tuning(t):
     return _default_tuning if t is None else t
 
 
+_bound = None   # the library whose functions the extension holds
+_ext = None
+
+
+def _native():
+    """dooms_amd._native (csrc/binding.cpp), the plain case of the entry points below in C++: each of its functions
+    returns what its namesake here does, a code of the library as an int, or None where the general path has to run."""
+    global _bound, _ext
+    L = _lib.lib()
+    if _bound is not L:
+        from . import _native as ext
+        ext.bind(*[ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in (
+            "mx_attn_prefill_ws", "mx_attn_decode", "mx_attn_decode_f32", "mx_attn_decode_rope", "mx_attn_prefill_rope_ws",
+            "mx_linear_workspace_bytes", "mx_linear", "mx_self_attention_workspace_bytes", "mx_self_attention")])
+        _bound, _ext = L, ext
+    return _ext
+
+
+def _result(r):
+    if type(r) is int:  # a code of the library other than OK
+        _lib.check(r)
+    return r
+
+
 def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
@@ -51,6 +78,11 @@ def prefill(q, k_cache, v_cache, *, n_head, n_head_kv, head_dim, p0=0, causal=Tr
     """mx_attn_prefill: q [n_q][>= n_head*hd], caches [n_kv][>= n_head_kv*hd]. Returns (out, lse or None).
     workspace: "auto" (sized and zeroed here) or a zeroed uint8 device tensor runs mx_attn_prefill_ws, which takes the
     split-KV kernel for chunks of few rows; None runs mx_attn_prefill."""
+    if _tuning(tuning) is None:
+        r = _native().prefill(q, k_cache, v_cache, n_head, n_head_kv, head_dim, p0, causal, n_kv, scale, out, lse, want_lse,
+                              workspace)
+        if r is not None:
+            return _result(r)
     _rows(q, "q"), _rows(k_cache, "k_cache"), _rows(v_cache, "v_cache")
     if k_cache.stride(0) != v_cache.stride(0):
         raise ValueError("k_cache and v_cache must share a row stride")
@@ -94,6 +126,11 @@ def decode(q, k_caches, v_caches, kv_len, *, n_head, n_head_kv, head_dim, n_q=1,
     """mx_attn_decode (float16 q) or mx_attn_decode_f32 (float32 q and output): q [batch*n_q][>= n_head*hd];
     k_caches/v_caches lists of [>= kv_len[b]][>= n_head_kv*hd] float16 tensors (entries may repeat); kv_len list of
     ints. Returns (out, lse or None)."""
+    if workspace is not None and _tuning(tuning) is None:
+        r = _native().decode(q, k_caches, v_caches, kv_len, n_head, n_head_kv, head_dim, n_q, causal, scale, out, lse, want_lse,
+                             workspace)
+        if r is not None:
+            return _result(r)
     batch = len(kv_len)
     if len(k_caches) != batch or len(v_caches) != batch:
         raise ValueError("k_caches, v_caches and kv_len must have one entry per sequence")
@@ -127,6 +164,11 @@ def decode_rope(qkv, k_caches, v_caches, kv_len, *, n_head, n_head_kv, head_dim,
     """mx_attn_decode_rope, the fused decode step: qkv f32 [batch][>= (n_head + 2 n_head_kv) hd] holds each sequence's
     new token unrotated (q | k | v); the token goes to position kv_len[b] - 1 of k_caches[b] / v_caches[b] (f16,
     written in place). Returns (out f32 [batch][n_head hd], lse or None)."""
+    if workspace is not None and _tuning(tuning) is None:
+        r = _native().decode_rope(qkv, k_caches, v_caches, kv_len, n_head, n_head_kv, head_dim, rope_mode, rope_base, scale, out,
+                                  lse, want_lse, workspace)
+        if r is not None:
+            return _result(r)
     batch = len(kv_len)
     if len(k_caches) != batch or len(v_caches) != batch:
         raise ValueError("k_caches, v_caches and kv_len must have one entry per sequence")
@@ -161,6 +203,11 @@ def prefill_rope(qkv, k_cache, v_cache, *, n_head, n_head_kv, head_dim, rope_mod
     and values are written (rotated, f16) into rows p0 .. of k_cache / v_cache, then the chunk attends.
     Returns (out f32 [n_q][n_head hd], lse or None). workspace ("auto" or a zeroed uint8 device tensor) runs
     mx_attn_prefill_rope_ws."""
+    if _tuning(tuning) is None:
+        r = _native().prefill_rope(qkv, k_cache, v_cache, n_head, n_head_kv, head_dim, rope_mode, rope_base, p0, causal, n_kv,
+                                   scale, out, lse, want_lse, workspace)
+        if r is not None:
+            return _result(r)
     _rows(qkv, "qkv", torch.float32), _rows(k_cache, "k_cache"), _rows(v_cache, "v_cache")
     if k_cache.stride(0) != v_cache.stride(0):
         raise ValueError("k_cache and v_cache must share a row stride")
@@ -191,6 +238,9 @@ def linear(x, weights, *, out=None, gamma=None, bias=None, eps=1e-5, accumulate=
     """mx_linear: x f32 [M][>= K]; weights: one f16 [N][K] tensor or a list of them (same shape, one launch);
     out: matching output tensor(s) (f32, or f16 with out_f16), created if None; gamma f32 [K] turns on the RMS norm;
     bias: f32 [N] tensor or list (None entries allowed). Returns the output tensor or list."""
+    r = _native().linear(x, weights, out, gamma, bias, eps, accumulate, out_f16)
+    if r is not None:
+        return _result(r)
     single = isinstance(weights, torch.Tensor)
     ws_list = [weights] if single else list(weights)
     _rows(x, "x", torch.float32)
@@ -231,6 +281,10 @@ _SA_DTYPES = {torch.float32: _lib.DTYPE_F32, torch.float16: _lib.DTYPE_F16, torc
 def self_attention(qkv, *, heads, scale=None, out=None, tuning=None):
     """mx_self_attention, the IR's SelfAttention op: qkv [B][N][3E] contiguous (f32, f16 or bf16) -> y [B][N][E] of the
     same dtype. scale defaults to head_dim^-0.5. The workspace (if the shape needs one) comes from torch's allocator."""
+    if _tuning(tuning) is None:
+        r = _native().self_attention(qkv, heads, scale, out)
+        if r is not None:
+            return _result(r)
     if not qkv.is_cuda:
         raise ValueError("qkv must be a device tensor")
     if qkv.dim() != 3 or not qkv.is_contiguous() or qkv.dtype not in _SA_DTYPES:

@@ -50,6 +50,26 @@ def build(verbose: bool = False, out: str = LIB, defines=()) -> str:
     return out
 
 
+EXT = os.path.join(PKG, "_native.so")
+
+
+def build_binding(out: str = EXT) -> str:
+    """The torch front end's extension (csrc/binding.cpp): host code only, against the headers of the torch in use."""
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(ROOT, "include"), os.path.join(root, "include"), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    rc, msg = _run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                    f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[x for d in inc for x in ("-isystem", d)],
+                    os.path.join(CSRC, "binding.cpp"), "-o", out + ".tmp", "-L", os.path.join(root, "lib"),
+                    "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"])
+    if rc != 0:
+        raise RuntimeError(f"g++ failed on the binding ({rc}):\n{msg}")
+    os.replace(out + ".tmp", out)
+    return out
+
+
 LIB_TRACE = os.path.join(os.path.dirname(LIB), "libmx_attn_trace.so")
 
 
@@ -79,6 +99,7 @@ def build_host_test() -> str:
 
 if __name__ == "__main__":
     print(build(verbose=True))
+    print(build_binding())
 
 
 SAN_DIR = os.path.join(ROOT, "tests", "cpp", "_san")
