@@ -132,6 +132,76 @@ DecodeShape decode_shape(const mx_attn_desc * d) {
     return s;
 }
 
+// Keys per split and waves per workgroup of one launch. Besides the plan of the comments above (the shortest splits, then
+// as few as kMaxSplits and the workgroup cap ask for), for one row tile at head dims 64 and 128 (swept over 117 shapes of 1
+// to 16 sequences, f16 and rotated rows; the plan below is within 0.7 % of the best split and waves on average, the
+// plan without it 5.2 %):
+//   * sequences of up to 256 keys (384 at head dim 64) whole, without a merge: 5 x 129 keys of 8 kv heads 6.13 -> 5.31 us,
+//     2 x 163 keys of 20 kv heads 5.25 -> 4.31 with 8 waves; at 388 keys of 20 heads the split is ahead (6.28 against 6.77);
+//   * head dim 64, several sequences: at most 16 splits, the most that one round of the merge folds (3 x 3096 keys of 2
+//     kv heads 8.20 -> 7.29);
+//   * one round of 8-wave workgroups on the CUs instead of several of 4 waves, whose starts and merges leave the memory
+//     idle: 16 ragged Llama-3-8B caches of 1025 to 8191 keys 61.9 -> 56.8, 4 of 1600 to 6800 22.7 -> 18.4. Launches
+//     that fit two 4-wave workgroups per CU with 128-key splits stay (16 x 396 keys 9.66 against 9.82). Off the
+//     XCD-mapped grid a ragged launch loses a few CUs to uneven dealing, so it is held to 208 workgroups, and splits past
+//     640 keys, where one workgroup too many on a CU costs the most, keep the 4-wave plan (16 Qwen2.5-7B caches of 1.9k
+//     to 10.5k keys: 49.6 us, 58.3 in one round).
+struct DecodePlan {
+    int64_t chunk;
+    int waves;
+};
+DecodePlan decode_plan(const mx_attn_desc & d, const int32_t * kv_len, int n_seq, int n_rowtiles, bool xcd) {
+    const mx_attn_tuning * t = d.tuning;
+    const int64_t quantum = mx::kDecodeChunkQuantum;
+    int64_t lmax = 0, lmin = INT64_MAX;
+    for (int i = 0; i < n_seq; i++) {
+        lmax = std::max<int64_t>(lmax, kv_len[i]);
+        lmin = std::min<int64_t>(lmin, kv_len[i]);
+    }
+    auto round_up = [&](int64_t x) { return (x + quantum - 1) / quantum * quantum; };
+    auto launch_wgs = [&](int64_t c) {
+        int64_t n = 0;
+        for (int i = 0; i < n_seq; i++) n += (kv_len[i] + c - 1) / c;
+        return n * d.n_head_kv * n_rowtiles;
+    };
+    // the smallest chunk, at least c, of at most cap workgroups (or the longest sequence whole): bisect over quanta
+    auto within = [&](int64_t c, int64_t cap) {
+        if (launch_wgs(c) <= cap) return c;
+        int64_t lo = c / quantum, hi = std::max(lo, round_up(lmax) / quantum);
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) / 2;
+            if (launch_wgs(mid * quantum) > cap) lo = mid + 1;
+            else hi = mid;
+        }
+        return lo * quantum;
+    };
+    if (t && t->decode_splits > 0) {
+        // the caller's split count (of the longest sequence): never more than one split per quantum of keys
+        const int64_t c = round_up((lmax + t->decode_splits - 1) / t->decode_splits);
+        return {c, decode_waves(t, c, launch_wgs(c))};
+    }
+    const bool tile = n_rowtiles == 1 && (d.head_dim == 64 || d.head_dim == 128) && !(t && t->decode_max_workgroups > 0);
+    const bool hd64 = d.head_dim == 64;
+    if (tile && lmax > quantum && lmax <= (hd64 ? 384 : 256))
+        return {round_up(lmax), t && t->decode_waves ? t->decode_waves : hd64 ? 8 : 4};
+    int64_t msplit = max_splits(&d, n_rowtiles, n_seq, lmax);
+    if (tile && hd64 && n_seq > 1 && lmax <= 16 * 640) msplit = 16;
+    int64_t chunk = round_up((lmax + msplit - 1) / msplit);
+    // A batch of at least 4 sequences of about one length (within 1.5x) and at least 4096 keys: at most 8 splits
+    // per sequence. A/B on one box, us per launch (8 splits of 4 waves against the plan of up to 32): Llama-3-8B
+    // 4 x 8192 keys 29.9 -> 26.4, 8 x 8192 51.9 -> 48.8, 16 x 8192 95.5 -> 90.1, 12 x 4096 42.3 -> 39.9,
+    // Qwen2.5-7B 8 x 4096 22.0 -> 17.7, 4 x 8192 19.5 -> 18.8, Qwen2.5-0.5B 8 x 4096 12.1 -> 9.8. Ragged batches
+    // keep the plan (Qwen2.5-7B 1.3k-7.3k x 16 35 -> 41.7 at 16 splits), as do shorter caches (4 x 2048: 11.5 -> 12.6).
+    if (n_seq >= 4 && lmin >= 4096 && 2 * lmax <= 3 * lmin) chunk = std::max(chunk, round_up((lmax + 7) / 8));
+    if (tile && !(xcd && chunk == quantum && launch_wgs(chunk) <= 512)) {
+        const bool even = xcd || n_seq == 1;  // every XCD gets the same number of workgroups
+        const int64_t c = within(chunk, even ? 256 : 208);
+        if (launch_wgs(c) <= 256 && (even || c <= 640)) return {c, decode_waves(t, c, launch_wgs(c))};
+    }
+    chunk = within(chunk, workgroup_cap(t));
+    return {chunk, decode_waves(t, chunk, launch_wgs(chunk))};
+}
+
 // Workspace layout: kMaxTilesPerLaunch split counters (one per (sequence of a launch, kv head, row tile), each on a
 // 256-byte line of its own) at a fixed place, then the partials. The counters must be zero when a call starts, and
 // every call leaves the ones it used at zero; the partials are left as they are. So the counter region has the same
@@ -524,43 +594,11 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
         const int64_t kv_bytes = kv_keys * d.kv_stride * 2 * 2;
         p.kv_nt = (p.xcd_heads && kv_bytes >= ((int64_t)16 << 20)) || kv_bytes >= ((int64_t)256 << 20);
         p.scale_log2 = d.scale * 1.4426950408889634f;
-        // split plan (see workgroup_cap)
-        const int64_t quantum = mx::kDecodeChunkQuantum;
-        int64_t lmax = 0;
-        for (int i = 0; i < n_seq; i++) lmax = std::max<int64_t>(lmax, kv_len[b0 + i]);
-        auto round_up = [&](int64_t x) { return (x + quantum - 1) / quantum * quantum; };
-        const int64_t msplit = max_splits(&d, s.n_rowtiles, n_seq, lmax);
-        int64_t chunk = round_up((lmax + msplit - 1) / msplit);
-        auto launch_wgs = [&](int64_t c) {
-            int64_t n = 0;
-            for (int i = 0; i < n_seq; i++) n += (kv_len[b0 + i] + c - 1) / c;
-            return n * d.n_head_kv * s.n_rowtiles;
-        };
-        const int64_t cap = workgroup_cap(d.tuning);
-        // A batch of at least 4 sequences of about one length (within 1.5x) and at least 4096 keys: at most 8 splits
-        // per sequence. A/B on one box, us per launch (8 splits of 4 waves against the plan of up to 32): Llama-3-8B
-        // 4 x 8192 keys 29.9 -> 26.4, 8 x 8192 51.9 -> 48.8, 16 x 8192 95.5 -> 90.1, 12 x 4096 42.3 -> 39.9,
-        // Qwen2.5-7B 8 x 4096 22.0 -> 17.7, 4 x 8192 19.5 -> 18.8, Qwen2.5-0.5B 8 x 4096 12.1 -> 9.8. Ragged batches
-        // keep the plan (Llama-3-8B 1.6k-6.8k keys x 4: 16.4 -> 19.9 at 8 splits; Qwen2.5-7B 1.3k-7.3k x 16 35 ->
-        // 41.7 at 16), as do shorter caches (4 x 2048: 11.5 -> 12.6).
-        int64_t lmin = lmax;
-        for (int i = 0; i < n_seq; i++) lmin = std::min<int64_t>(lmin, kv_len[b0 + i]);
-        const bool uniform = n_seq >= 4 && lmin >= 4096 && 2 * lmax <= 3 * lmin;
-        if (uniform && !(d.tuning && d.tuning->decode_splits > 0)) chunk = std::max(chunk, round_up((lmax + 7) / 8));
-        if (d.tuning && d.tuning->decode_splits > 0) {
-            // the caller's split count (of the longest sequence): never more than one split per quantum of keys
-            chunk = round_up((lmax + d.tuning->decode_splits - 1) / d.tuning->decode_splits);
-        } else if (launch_wgs(chunk) > cap) {  // smallest chunk within the cap: bisect over multiples of the quantum
-            int64_t lo = chunk / quantum, hi = round_up(lmax) / quantum;
-            while (lo < hi) {
-                const int64_t mid = (lo + hi) / 2;
-                if (launch_wgs(mid * quantum) > cap) lo = mid + 1;
-                else hi = mid;
-            }
-            chunk = lo * quantum;
-        }
+        const DecodePlan plan = decode_plan(d, kv_len + b0, n_seq, s.n_rowtiles, p.xcd_heads);
+        const int64_t chunk = plan.chunk;
         p.chunk = (int32_t)std::min<int64_t>(chunk, INT32_MAX / 2);
         p.max_split = 1;
+        int32_t xcd0 = 0;
         for (int i = 0; i < n_seq; i++) {
             const int32_t n = kv_len[b0 + i];
             p.seq[i].k = static_cast<const mx::half_t *>(k_caches[b0 + i]);
@@ -568,8 +606,10 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
             p.seq[i].len = n;
             p.seq[i].n_split = (int32_t)((n + p.chunk - 1) / p.chunk);
             p.max_split = std::max(p.max_split, p.seq[i].n_split);
+            p.seq[i].xcd0 = xcd0;
+            xcd0 = (xcd0 + p.seq[i].n_split * d.n_head_kv) % 8;
         }
-        for (int i = n_seq; i < mx::kMaxSeqPerLaunch; i++) p.seq[i] = mx::DecodeSeq{nullptr, nullptr, 0, 0};
+        for (int i = n_seq; i < mx::kMaxSeqPerLaunch; i++) p.seq[i] = mx::DecodeSeq{};
         // The XCD-mapped grid (partials published into one XCD's L2) also for one short sequence whatever its kv heads:
         // a few splits over at most 4 MB of keys and values, where the merge chain outweighs the stream, which the
         // grid concentrates on min(kv heads, 8) XCDs. Qwen2.5-0.5B at 513 keys 4.99 -> 4.50 us per launch, Whisper
@@ -577,8 +617,7 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
         // 2048 keys, two XCDs streaming) measured 5.87 -> 6.02, Whisper cross-attention (12 splits, 7.7 MB) no gain.
         if (n_seq == 1 && p.max_split <= 8 && kv_bytes <= ((int64_t)4 << 20)) p.xcd_heads = 1;
         if (p.max_split > 32) p.xcd_heads = 0;  // the XCD-local counter counts at most 63 splits per XCD field
-        const int waves = decode_waves(d.tuning, p.chunk, launch_wgs(p.chunk));
-        if (int32_t rc = hip_status(mx::launch_decode(p, n_seq, d.head_dim, s.rt, waves, st), "decode launch")) return rc;
+        if (int32_t rc = hip_status(mx::launch_decode(p, n_seq, d.head_dim, s.rt, plan.waves, st), "decode launch")) return rc;
     }
     return MX_ATTN_OK;
 }

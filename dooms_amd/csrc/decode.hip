@@ -235,8 +235,11 @@ __device__ __forceinline__ void merge_wide(const DecodeParams & p, const float *
 // from the q|k|v row; q and the new key are rotated for position kv_len - 1 and rounded to half, the new key and value
 // are used from registers for that position and written into the caches by the one workgroup whose split holds it.
 // NT: the keys and values are loaded non-temporally (p.kv_nt: a launch whose K/V stream from HBM once).
+// Head dim 128: two waves per SIMD at least. Without the bound the f32 variants of 4 waves took 288 registers, one wave
+// per SIMD, and a launch of more workgroups than CUs ran them in twice the rounds.
 template <int HD, int RT, bool F32, int NW, bool NT = false>
-__global__ __launch_bounds__(NW * kWave) void decode_kernel(DecodeParams p) {
+__global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(HD == 128 || NW == 8 ? 2 : 1)))
+void decode_kernel(DecodeParams p) {
     using B = KvBlock<HD>;
     constexpr int KS = B::KS, LPR = B::LPR, KPL = B::KPL, NLV = B::NLV;
 
@@ -259,13 +262,13 @@ __global__ __launch_bounds__(NW * kWave) void decode_kernel(DecodeParams p) {
     const int bl = blockIdx.y;
     const half_t * seq_k = p.seq[bl].k;
     const half_t * seq_v = p.seq[bl].v;
-    int32_t L = p.seq[bl].len, n_split = p.seq[bl].n_split;
+    int32_t L = p.seq[bl].len, n_split = p.seq[bl].n_split, xcd0 = p.seq[bl].xcd0;
     uint32_t T = p.n_rowtiles;
     int32_t max_split = p.max_split, n_head_kv = p.n_head_kv, chunk = p.chunk, G = p.group, seq0 = p.seq0, n_q = p.n_q;
     int32_t rows = p.rows, causal = p.causal, xcd_heads = p.xcd_heads;
     int64_t q_stride = p.q_stride, kv_stride = p.kv_stride;
     const half_t * qp = p.q;
-    asm volatile("" : "+s"(seq_k), "+s"(seq_v), "+s"(L), "+s"(n_split), "+s"(T), "+s"(max_split), "+s"(n_head_kv),
+    asm volatile("" : "+s"(seq_k), "+s"(seq_v), "+s"(L), "+s"(n_split), "+s"(xcd0), "+s"(T), "+s"(max_split), "+s"(n_head_kv),
                  "+s"(chunk), "+s"(G), "+s"(seq0), "+s"(n_q), "+s"(rows), "+s"(causal), "+s"(xcd_heads), "+s"(q_stride),
                  "+s"(kv_stride), "+s"(qp));
     // the fused step's own arguments likewise (fetched behind branches they cost dependent scalar round trips ahead
@@ -299,9 +302,13 @@ __global__ __launch_bounds__(NW * kWave) void decode_kernel(DecodeParams p) {
         s = u % max_split;
         g = (u / max_split) * 8 + id % 8;
     } else {
-        const uint32_t grp = u * 8 + id % 8;  // (split, kv head) group of the sequence
-        s = grp % max_split;
-        g = grp / max_split;
+        // (split, kv head) group of the sequence, its first on the XCD after the previous sequence's last: the live
+        // workgroups of a ragged batch spread evenly over the XCDs (numbered by the longest sequence's splits, those
+        // of shorter ones fell on a few XCDs, whose CUs then took two rounds: 8 sequences of 1116 to 4061 keys, 4 kv heads,
+        // 236 workgroups of 8 waves 20.9 us against 15.9 for 180)
+        const uint32_t grp = u * 8 + (id - (uint32_t)xcd0) % 8;
+        s = grp % n_split;
+        g = grp / n_split;
     }
     if (g >= n_head_kv) return;  // padding of the grid to whole XCD rounds
     if (s >= n_split) return;    // uniform over the workgroup, before any barrier

@@ -25,6 +25,8 @@ struct DecodeSeq {
     const half_t * v;
     int32_t len;      // keys in the cache
     int32_t n_split;  // splits of `chunk` keys covering them
+    int32_t xcd0;     // the XCD of its first workgroup (without xcd_heads): where the sequence before it ended
+    int32_t pad;
 };
 
 struct DecodeParams {

@@ -320,3 +320,27 @@ def test_workspace_shared_across_shapes(device):
         torch.cuda.synchronize()
         assert torch.equal(got.view(torch.int16), ref.view(torch.int16)), f"{nh}/{nkv} {lens} n_q {nq}"
         assert torch.equal(gl.view(torch.int32), rl.view(torch.int32))
+
+
+@pytest.mark.parametrize("H,G,hd", [(4, 4, 64), (20, 20, 64), (14, 2, 64), (32, 8, 128), (12, 4, 128), (4, 1, 256)])
+@pytest.mark.parametrize("lens", [[128], [129], [256, 130, 7], [257, 1], [384, 129, 300, 2], [385, 128], [2049, 300],
+                                  [2600] + [100 + 37 * i for i in range(19)], [5000, 4999, 4600, 4200, 4100],
+                                  [1100 - 50 * i for i in range(16)]])
+def test_plan_edges(device, H, G, hd, lens):
+    """Lengths at the edges of the split plan (whole sequences, one merge round, one round of 8-wave workgroups, the
+    workgroup cap), ragged so that the sequences' workgroups start on different XCDs: f16 and f32 rows against f64."""
+    g = torch.Generator(device=device)
+    g.manual_seed(sum(lens) + hd)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=device)
+    q = rnd(len(lens), H * hd)
+    ks, vs = [rnd(n, G * hd).half() for n in lens], [rnd(n, G * hd).half() for n in lens]
+    refs, lses = [], []
+    for b, n in enumerate(lens):
+        qq = q[b].half().double().view(G, H // G, hd)
+        s = torch.stack([qq[i] @ ks[b].double().view(n, G, hd)[:, i].T for i in range(G)]) / hd ** 0.5
+        refs.append(torch.stack([torch.softmax(s[i], 1) @ vs[b].double().view(n, G, hd)[:, i] for i in range(G)]).flatten())
+        lses.append(torch.logsumexp(s, 2).flatten())
+    ref, rl = torch.stack(refs).cpu().numpy(), torch.stack(lses).cpu().numpy()
+    for dt in (torch.float16, torch.float32):
+        out, lse = A.decode(q.to(dt), ks, vs, lens, n_head=H, n_head_kv=G, head_dim=hd, want_lse=True)
+        assert_close(out.float().cpu().numpy(), ref, hd, f"{lens} {dt}", lse.cpu().numpy(), rl)
