@@ -382,10 +382,15 @@ __global__ __launch_bounds__(kGemvMaxWaves * kWave) void gemv_kernel(LinearParam
 // 256 x 256 halves the bytes per product (and 128 x 64 per wave cuts the LDS reads per product by a quarter). The
 // tiles go from HBM/L2 straight into LDS (global_load_lds_dwordx4: lane l's 16 bytes land at byte 16 l of the
 // instruction's 1 KB destination), two buffers (the loads of step s + 1 in flight while step s multiplies), no
-// registers in between. An operand tile (256 rows x 64 columns) is two column groups of 16 blocks of 16 rows x 64
-// bytes, one load instruction each; 16-byte chunk c of row r sits at 16 (c ^ ((r % 16) / 4)) within its row's 64 bytes,
-// so the 16-byte operand reads of 16 consecutive rows at one chunk land on 16 distinct 4-bank groups. 128 KB of LDS:
-// one workgroup per CU, two waves per SIMD.
+// registers in between. A load covers 8 rows x 128 bytes, whole cache lines: in pieces of 64 bytes every line came to
+// the CU twice. 16-byte chunk c of row r sits at 16 (c ^ (r / 2 % 8)) within its row's 128 bytes, so the 16-byte operand
+// reads of 16 consecutive rows at one chunk land on 16 distinct 4-bank groups. 128 KB of LDS: one workgroup per CU,
+// two waves per SIMD, which take turns (below). The load path bounds it: without the loads 2048 x 6144 x 4096 takes
+// 102 us instead of 130, without most of the products 105, without half of the operand reads no less. Against one barrier per
+// step, both waves of a SIMD in step and 64-byte pieces (us, staging included, one box): 2048 x 6144 x 4096 140 -> 130,
+// 4096 x 4096 x 4096 175 -> 158, 8 products of 1500 x 1280 x 1280 62.8 -> 55.7, 1024 x 14336 x 4096 150 -> 136, 3000 x 4096 x
+// 14336 445 -> 392. The raised wave priority around the products, the loads all in the first phase, spread over all
+// four or ahead of the operand reads, and phases of two slices measured 1 to 10 % slower.
 // BN = 192 (256 x 192, 8 waves of 64 x 96) serves products whose 256 x 256 tiles would leave CUs idle.
 constexpr int kBM = 256;
 constexpr int kGemmCUs = 256;
@@ -394,17 +399,12 @@ constexpr int kBigWaves = 8, kBigThreads = kBigWaves * kWave;
 template <bool OUT16, int BN, int WC>
 __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
     constexpr int kBN = BN, kBK = 64;
-    constexpr int kBigBufs = 2;
-    constexpr int kBigLoads = kBM * kBK * 2 / 1024 / kBigWaves;  // 1 KB direct loads of A per wave and step
-    constexpr int RA = kBM / 16, RBB = BN / 16;                  // 16-row blocks per chunk group of A and of B
+    constexpr int kBlocks = (kBM + BN) / 8;                  // 1 KB blocks (8 rows x 128 bytes) of a step's tiles
+    constexpr int Loads = kBlocks / kBigWaves;               // direct loads per wave and step
     constexpr int WN = BN / WC, WM = kBigWaves / WN;         // waves along N and along M
     constexpr int kBigMI = kBM / WM / 32, kBigNJ = WC / 32;  // 32 x 32 MFMA tiles per wave
-    constexpr int BBlocks = BN * kBK * 2 / 1024;             // 1 KB blocks of a step's B tile
-    constexpr int BLoads = (BBlocks + kBigWaves - 1) / kBigWaves;  // direct loads of B per wave and step; past the
-                                                                   // tile's blocks a wave reloads one it already loads
-    static_assert(BLoads >= 1 && kBigMI >= 1 && WN * WM == kBigWaves, "whole loads and tiles per wave");
-    __shared__ __attribute__((aligned(1024))) half_t xs[kBigBufs][kBM * kBK];
-    __shared__ __attribute__((aligned(1024))) half_t ws[kBigBufs][BN * kBK];
+    static_assert(kBlocks % kBigWaves == 0 && kBigMI >= 1 && WN * WM == kBigWaves, "whole loads and tiles per wave");
+    __shared__ __attribute__((aligned(1024))) half_t sm[2][(kBM + BN) * kBK];  // A's rows, then B's
     const int n_tiles = (p.N + kBN - 1) / kBN, m_tiles = (p.M + kBM - 1) / kBM;
     // consecutive work items share a weight tile (different token tiles); contiguous ranges per XCD
     const uint32_t t = xcd_remap(blockIdx.x, (uint32_t)(p.count * n_tiles * m_tiles));
@@ -414,40 +414,28 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
     const int l32 = lane % 32, hi = lane / 32;
 
     // Each lane's source bytes relative to the step's first column are fixed: rows past M (N) repeat the last row.
-    // The staged rows are kp halves apart (K rounded up to 64, zero-padded); the weight rows K halves apart.
-    const int kp = (p.K + 63) / 64 * 64;
-    const char * a_base = reinterpret_cast<const char *>(p.xh + (int64_t)m0 * kp);
+    // K is a multiple of 64 here, so the staged rows are K halves apart, as the weight rows. Lane l of block j fills
+    // position l % 8 of the tile's row 8 j + l / 8 with 16-byte chunk (l % 8) ^ (row / 2 % 8).
+    const char * a_base = reinterpret_cast<const char *>(p.xh + (int64_t)m0 * p.K);
     const char * b_base = reinterpret_cast<const char *>(p.w[mi] + (int64_t)n0 * p.K);
-    uint32_t a_off[kBigLoads], b_off[BLoads];
-    const int c = (lane % 4) ^ (lane / 16);  // the chunk a lane fetches for position lane % 4 of its row's 64 bytes
-    // block j of a tile: chunk group j / R (64-byte column group), rows 16 (j % R) ..
+    uint32_t off[Loads];
 #pragma unroll
-    for (int i = 0; i < kBigLoads; i++) {
-        const int j = i * kBigWaves + wave;
-        const int row = 16 * (j % RA) + lane / 4;  // the row this lane fills
-        a_off[i] = (uint32_t)(min(m0 + row, p.M - 1) - m0) * kp * 2 + 64 * (j / RA) + 16 * c;
+    for (int i = 0; i < Loads; i++) {
+        const int row = 8 * (i * kBigWaves + wave) + lane / 8;
+        const int r = row < kBM ? gemm_load_row(m0, row, p.M) - m0 : gemm_load_row(n0, row - kBM, p.N) - n0;
+        off[i] = (uint32_t)r * (uint32_t)p.K * 2 + 16 * ((lane % 8) ^ ((row >> 1) & 7));
     }
-#pragma unroll
-    for (int i = 0; i < BLoads; i++) {
-        const int j = i * kBigWaves + wave, jb = j < BBlocks ? j : j - kBigWaves;  // (identical bytes written twice)
-        const int row = 16 * (jb % RBB) + lane / 4;
-        b_off[i] = (uint32_t)(min(n0 + row, p.N - 1) - n0) * p.K * 2 + 64 * (jb / RBB) + 16 * c;
-    }
-    auto issue = [&](int step, int buf) __attribute__((always_inline)) {
+    // loads I0 .. I1 - 1 of a step
+    auto issue = [&](int step, auto I0C, auto I1C) __attribute__((always_inline)) {
         const int64_t k0 = (int64_t)step * kBK * 2;  // bytes
-        // A and B loads interleaved
-#pragma unroll
-        for (int i = 0; i < kBigLoads; i++) {
-            __builtin_amdgcn_global_load_lds(a_base + k0 + a_off[i],
-                                             (__attribute__((address_space(3))) void *)&xs[buf][512 * (i * kBigWaves + wave)],
-                                             16, 0, 0);
-            if (i < BLoads) {
-                const int j = i * kBigWaves + wave, jb = j < BBlocks ? j : j - kBigWaves;
-                __builtin_amdgcn_global_load_lds(b_base + k0 + b_off[i],
-                                                 (__attribute__((address_space(3))) void *)&ws[buf][512 * jb], 16, 0, 0);
-            }
-        }
+        static_for<decltype(I0C)::value, decltype(I1C)::value>([&](auto I) __attribute__((always_inline)) {
+            constexpr int i = decltype(I)::value;
+            const int j = i * kBigWaves + wave;
+            __builtin_amdgcn_global_load_lds((i * kBigWaves < kBM / 8 ? a_base : b_base) + k0 + off[i],
+                                             (__attribute__((address_space(3))) void *)&sm[step & 1][512 * j], 16, 0, 0);
+        });
     };
+    static_assert(kBM / 8 % kBigWaves == 0, "a load is of A or of B for every wave");
 
     float16_t acc[kBigMI][kBigNJ];
 #pragma unroll
@@ -457,63 +445,76 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
 
-    // this wave's block: rows (256 / WM) wm + 32 i + l32 of A, columns 64 wn + 32 j + l32 (rows of B); fragment
-    // (row, chunk 2 ks + hi) at halves 512 (row / 16) + 32 (row % 16) + 8 ((2 ks + hi) ^ ((row % 16) / 4))
+    // this wave's block: rows (256 / WM) wm + 32 i + l32 of A, columns WC wn + 32 j + l32 (rows of B); fragment (row,
+    // chunk 2 ks + hi) at byte 128 row + 16 ((2 ks + hi) ^ (row / 2 % 8))
     const int wm = wave / WN, wn = wave % WN;
-    int rd[2];
+    uint32_t rd[4];
 #pragma unroll
-    for (int ks = 0; ks < 2; ks++) rd[ks] = 512 * (l32 / 16) + 32 * (l32 % 16) + 8 * ((2 * ks + hi) ^ ((l32 % 16) / 4));
-    const int nk = p.K / kBK;
-#pragma unroll
-    for (int a = 0; a < kBigBufs - 1; a++)
-        if (a < nk) issue(a, a);
-    for (int s = 0; s < nk; s++) {
-        const int buf = s % kBigBufs;
-        // this wave's loads of step s are complete, then every wave's are; the buffer refilled below was last read in
-        // step s - 1
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    for (int ks = 0; ks < 4; ks++) rd[ks] = 128 * l32 + 16 * ((2 * ks + hi) ^ ((l32 >> 1) & 7));
+    const uint32_t sm0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) half_t *)sm[0];
+    auto barrier = []() __attribute__((always_inline)) {
         asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
         asm volatile("" ::: "memory");
-        if (s + kBigBufs - 1 < nk) issue(s + kBigBufs - 1, (s + kBigBufs - 1) % kBigBufs);
-        // the operand reads as inline asm (the compiler cannot tell them from the direct loads in flight, and would
-        // wait for those), all of the step's in flight, the products of each 16-column slice behind their reads
-        const uint32_t xa = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) half_t *)xs[buf] + 2 * 32 * (kBM / WM) * wm;
-        const uint32_t wa = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) half_t *)ws[buf] + 2 * 32 * WC * wn;
-        // 4 slices of 16 columns: slices s + 1's reads in flight behind slice s's products (at most 2 slices of
-        // reads outstanding, within the 15 that lgkmcnt counts); the waits are ordered by sched_barrier
-        constexpr int R = kBigMI + kBigNJ;  // reads per slice
-        u32x4 fa[4][kBigMI], fb[4][kBigNJ];
-        auto reads = [&](auto KS) __attribute__((always_inline)) {
-            constexpr int ks = decltype(KS)::value;
-            const uint32_t ra_ = xa + 2 * (rd[ks % 2] + 512 * RA * (ks / 2)), rb_ = wa + 2 * (rd[ks % 2] + 512 * RBB * (ks / 2));
-            static_for<0, kBigMI>([&](auto I) __attribute__((always_inline)) {
-                u32x4 r;
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(ra_), "i"(2 * 1024 * decltype(I)::value));
-                fa[ks][decltype(I)::value] = r;
-            });
-            static_for<0, kBigNJ>([&](auto J) __attribute__((always_inline)) {
-                u32x4 r;
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(rb_), "i"(2 * 1024 * decltype(J)::value));
-                fb[ks][decltype(J)::value] = r;
-            });
-        };
-        reads(std::integral_constant<int, 0>{});
-        reads(std::integral_constant<int, 1>{});
+    };
+    const int nk = p.K / kBK;
+    using I0 = std::integral_constant<int, 0>;
+    using IH = std::integral_constant<int, Loads / 2>;
+    using IE = std::integral_constant<int, Loads>;
+    issue(0, I0{}, IE{});
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    barrier();
+    // Waves 4 .. 7 run half a phase behind waves 0 .. 3: of the two waves of a SIMD one multiplies while the other reads its
+    // operands and issues loads. A phase is a 16-column slice of a step: the slice's operand reads (and in phases 0 and
+    // 1 the next step's loads), a barrier, its products, a barrier.
+    const bool behind = wave >= kBigWaves / 2;
+    if (behind) barrier();
+    for (int s = 0; s < nk; s++) {
+        const uint32_t xa = sm0 + (uint32_t)(s & 1) * ((kBM + BN) * kBK * 2) + 128 * (kBM / WM) * wm;
+        const uint32_t wa = sm0 + (uint32_t)(s & 1) * ((kBM + BN) * kBK * 2) + 128 * (kBM + WC * wn);
         static_for<0, 4>([&](auto KS) __attribute__((always_inline)) {
             constexpr int ks = decltype(KS)::value;
-            if constexpr (ks < 3) asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(R) : "memory");
-            else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_sched_barrier(0);
+            // the operand reads as inline asm (the compiler cannot tell them from the direct loads in flight, and would
+            // wait for those)
+            u32x4 fa[kBigMI], fb[kBigNJ];
+            static_for<0, kBigNJ>([&](auto J) __attribute__((always_inline)) {
+                u32x4 r;
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(wa + rd[ks]), "i"(4096 * decltype(J)::value));
+                fb[decltype(J)::value] = r;
+            });
+            static_for<0, kBigMI>([&](auto I) __attribute__((always_inline)) {
+                u32x4 r;
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(xa + rd[ks]), "i"(4096 * decltype(I)::value));
+                fa[decltype(I)::value] = r;
+            });
+            // the other buffer was last read in phase 3 of step s - 1; every wave's reads of that phase were complete
+            // before the barrier that ended it (lgkmcnt(0) below)
+            if (s + 1 < nk) {
+                if constexpr (ks == 0) issue(s + 1, I0{}, IH{});
+                if constexpr (ks == 1) issue(s + 1, IH{}, IE{});
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            // the next step's loads are complete before the barrier after which waves 0 .. 3 read them: for waves 4 .. 7
+            // that is this one, for waves 0 .. 3 the one that ends the phase
+            if constexpr (ks == 3) {
+                if (behind) __builtin_amdgcn_s_waitcnt(0x0F70);
+            }
+            barrier();
+            
 #pragma unroll
             for (int i = 0; i < kBigMI; i++)
 #pragma unroll
-                for (int j = 0; j < kBigNJ; j++)
-                    acc[i][j] = mfma32x32x16(as_half8(fa[ks][i]), as_half8(fb[ks][j]), acc[i][j]);
-            __builtin_amdgcn_sched_barrier(0);
-            if constexpr (ks + 2 < 4) reads(std::integral_constant<int, ks + 2>{});
+                for (int j = 0; j < kBigNJ; j++) acc[i][j] = mfma32x32x16(as_half8(fa[i]), as_half8(fb[j]), acc[i][j]);
+            
+            if constexpr (ks == 3) {
+                if (!behind) __builtin_amdgcn_s_waitcnt(0x0F70);
+            }
+            barrier();
         });
     }
+    if (!behind) barrier();  // the barrier that the other half began with
 
     // lane holds Y[m0 + (256 / WM) wm + 32 i + 8 (v / 4) + 4 hi + v % 4][n0 + WC wn + 32 j + l32]
 #pragma unroll
@@ -790,8 +791,8 @@ const GemmCfg & gemm_cfg(int c) {
         MX_SPLIT(128, 64, 2, 128, 3, 1, 0.421f, 0.f, 1.094f, 0.765f, 0.348f),
         MX_SPLIT(128, 128, 2, 64, 4, 1, 0.640f, 0.f, 2.207f, 0.930f, 0.203f),
         MX_SPLIT(128, 128, 2, 64, 2, 2, 0.887f, 1.078f, 0.f, 1.092f, 0.306f),
-        {256, 192, 64, kBigThreads, 1, 1.279f, 0.f, 8.563f, 0.f, 0.f, gemm_w192_kernel<false>, gemm_w192_kernel<true>},
-        {256, 256, 64, kBigThreads, 1, 1.609f, 0.f, 10.664f, 0.f, 0.f, gemm_big_kernel<false>, gemm_big_kernel<true>},
+        {256, 192, 64, kBigThreads, 1, 1.243f, 0.f, 5.946f, 0.f, 0.f, gemm_w192_kernel<false>, gemm_w192_kernel<true>},
+        {256, 256, 64, kBigThreads, 1, 1.426f, 0.f, 8.941f, 0.f, 0.f, gemm_big_kernel<false>, gemm_big_kernel<true>},
     };
 #undef MX_SPLIT
     return cfgs[c];
