@@ -391,6 +391,13 @@ int prefill_choose_plan(const mx_attn_desc & d, int64_t n_kv, bool sk_ok) {
     const int64_t wg8 = (int64_t)((d.n_q + 255) / 256) * d.n_head;
     if (d.head_dim == 64) {
         if (sk_ok && n_kv >= 2 * (int64_t)d.n_q && wg8 < kSkRanges && prefill_sk_plan(d, n_kv, 8).ranges > 0) return 8;
+        // where the 64-row workgroups leave half the CUs idle: 32-row ones, four waves sharing a row tile's keys, which
+        // halves each wave's chain of blocks again (Qwen2.5-0.5B, us: 512 tokens 10.05 -> 9.4, 150 rows behind 1000
+        // 15.8 -> 13.0, 400 behind 400 13.7 -> 12.5, 300 behind 3000 34.2 -> 28.4); below 512 keys a prompt's first
+        // tiles have too few blocks for four waves (300 tokens 8.85 -> 9.2)
+        if (plan == 2 && (n_kv >= 8 * mx::kPrefillSkKeys || d.p0 >= 3 * mx::kPrefillSkKeys) &&
+            (int64_t)((d.n_q + 63) / 64) * d.n_head <= 128)
+            return 1;
         return plan == 2 ? 2 : 4;
     }
     if (d.head_dim == 128) {

@@ -96,7 +96,7 @@ struct PrefillParams {
     // the IR self-attention's rows read in place (kernel variants for f32, bf16 or f16 rows): head_dim of the rows
     // (<= the kernel's, a multiple of 8; columns past it are zeros) and the elements between consecutive heads
     int32_t hdv, head_stride;
-    int32_t plan;  // workgroup plan fixed by the caller (8, 4 or 2), or 0: prefill_plan's choice
+    int32_t plan;  // workgroup plan fixed by the caller (8, 4, 2 or 1), or 0: prefill_plan's choice
     // Stream-K launch (plan 8, one problem; sk_ranges 0 otherwise): sk_ranges workgroups each take an equal range of
     // the launch's sk_total (query tile, 64-key block) units; a tile split between ranges is merged through sk_part
     // (2 slots of kPrefillSlotFloats<HD> per range) and sk_counters (one uint32 per tile, zero between calls).

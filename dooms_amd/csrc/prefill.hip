@@ -85,8 +85,9 @@ constexpr bool prefill_dl() {
 
 template <int HD, int KSP, int W>
 struct PrefillSmem<HD, KSP, true, W> {
-    // 8 waves (one workgroup per CU): 3; 4 waves: 4 at head dim 64, 2 at 128 (64 KB, two workgroups per CU)
-    static constexpr int NBUF = W == 8 ? 3 : (HD == 64 ? 4 : 2);
+    // 8 waves (one workgroup per CU): 3; 4 waves: 4 at head dim 64 (2 with four key quarters: 64 KB steps), 2 at 128
+    // (64 KB, two workgroups per CU)
+    static constexpr int NBUF = W == 8 ? 3 : (HD == 64 && KSP <= 2 ? 4 : 2);
     half_t k[NBUF][KSP * kBK * HD];
     half_t v[NBUF][KSP * kBK * HD];
 };
@@ -818,13 +819,14 @@ void prefill_sk_kernel(PrefillParams p) {
 // K/V bytes per key) and with the 128-row workgroups filling at most a quarter of the CUs, the split pays from 128
 // keys: Qwen2.5-0.5B prompts of 128, 256 and 384 tokens 6.06 -> 5.9, 8.2 -> 7.5 and 10.0 -> 9.3 us per layer (a
 // 448-token prompt of 20 heads, 80 such workgroups, ran 9 % slower split).
-// Plans: 8 = 8 waves x 32 rows, 4 = 4 waves x 32 rows, 2 = 4 waves over 2 row tiles x 2 key halves (64 rows).
+// Plans: 8 = 8 waves x 32 rows, 4 = 4 waves x 32 rows, 2 = 4 waves over 2 row tiles x 2 key halves (64 rows), 1 = 4 waves
+// over the key quarters of one row tile (32 rows, head dim 64, chosen by the caller only).
 constexpr int kCUs = 256;
 int prefill_plan(int n_q, int n_head, int n_kv, int head_dim, int forced) {
     // head dim 256: 4 waves of 32 rows, one workgroup per CU (the K/V double buffer takes 141 KB of LDS; 8 waves or
     // the key-split plan would not fit the registers or the LDS)
     if (head_dim == 256) return 4;
-    if (forced == 2 || forced == 4 || forced == 8) return forced;
+    if (forced == 1 || forced == 2 || forced == 4 || forced == 8) return forced;
     const int64_t wg8 = (int64_t)((n_q + 255) / 256) * n_head, wg4 = (int64_t)((n_q + 127) / 128) * n_head;
     if (2 * wg4 <= kCUs && n_kv >= 8 * kBK) return 2;
     if (4 * wg4 <= kCUs && head_dim <= 64 && n_kv >= 2 * kBK) return 2;
@@ -938,7 +940,10 @@ void launch_prefill_r(const PrefillParams & p, int plan, int n_batch, hipStream_
     const dim3 grid((uint32_t)p.n_qtiles * p.n_head, (uint32_t)n_batch);
     if (plan == 8) hipLaunchKernelGGL((prefill_kernel<HD, POS, 8, ROPE, 1, SA>), grid, dim3(8 * kWave), 0, stream, p);
     else if (plan == 4) hipLaunchKernelGGL((prefill_kernel<HD, POS, 4, ROPE, 1, SA>), grid, dim3(4 * kWave), 0, stream, p);
-    else hipLaunchKernelGGL((prefill_kernel<HD, POS, 4, ROPE, 2, SA>), grid, dim3(4 * kWave), 0, stream, p);
+    else if constexpr (HD == 64 && SA == 0) {
+        if (plan == 1) hipLaunchKernelGGL((prefill_kernel<HD, POS, 4, ROPE, 4, SA>), grid, dim3(4 * kWave), 0, stream, p);
+        else hipLaunchKernelGGL((prefill_kernel<HD, POS, 4, ROPE, 2, SA>), grid, dim3(4 * kWave), 0, stream, p);
+    } else hipLaunchKernelGGL((prefill_kernel<HD, POS, 4, ROPE, 2, SA>), grid, dim3(4 * kWave), 0, stream, p);
 }
 
 template <int HD, bool POS>

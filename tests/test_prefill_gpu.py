@@ -257,3 +257,29 @@ def test_prefill_ws_noncausal_and_extra_keys(device):
         for out, lse in ((a, la), (b, lb)):
             assert_close(out.cpu().numpy().astype(np.float64)[:, cols], ro, hd, f"causal={causal}",
                          lse.cpu().numpy()[:, [0, 6, 7, 27]], rl)
+
+
+@pytest.mark.parametrize("H,G", [(14, 2), (4, 4)])
+@pytest.mark.parametrize("n_q,p0", [(512, 0), (513, 0), (575, 0), (65, 192), (64, 448), (33, 700), (300, 213), (1, 1000), (129, 3001)])
+def test_four_key_quarters(device, H, G, n_q, p0):
+    """Few workgroups at head dim 64: 32-row workgroups whose four waves take a row tile's 64-key blocks in turn; row and
+    key counts at the edges of the tiles, of the 256-key steps and of a wave's block, plain and rotated rows against f64."""
+    hd, n = 64, n_q + p0
+    g = torch.Generator(device=device)
+    g.manual_seed(n_q + p0 + H)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=device)
+    q, k, v = rnd(n_q, H * hd).half(), rnd(n, G * hd).half(), rnd(n, G * hd).half()
+    qq = q.double().view(n_q, H, hd)
+    kk, vv = (x.double().view(n, G, hd).repeat_interleave(H // G, 1) for x in (k, v))
+    hide = torch.arange(n, device=device)[None, :] > p0 + torch.arange(n_q, device=device)[:, None]
+    ref, rl = [], []
+    for h in range(H):
+        s = (qq[:, h] @ kk[:, h].T / 8).masked_fill(hide, float("-inf"))
+        ref.append(torch.softmax(s, 1) @ vv[:, h])
+        rl.append(torch.logsumexp(s, 1))
+    ref, rl = torch.cat(ref, 1).cpu().numpy(), torch.stack(rl, 1).cpu().numpy()
+    out, lse = A.prefill(q, k, v, n_head=H, n_head_kv=G, head_dim=hd, p0=p0, want_lse=True)
+    assert_close(out.float().cpu().numpy(), ref, hd, f"{n_q} rows at {p0}", lse.cpu().numpy(), rl)
+    qkv = torch.cat([q.float(), k[p0:].float(), v[p0:].float()], 1)
+    out, lse = A.prefill_rope(qkv, k.clone(), v.clone(), n_head=H, n_head_kv=G, head_dim=hd, p0=p0, rope_mode=2, want_lse=True)
+    assert_close(out.cpu().numpy(), ref, hd, f"{n_q} f32 rows at {p0}", lse.cpu().numpy(), rl)
