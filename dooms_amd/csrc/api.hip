@@ -141,11 +141,12 @@ DecodeShape decode_shape(const mx_attn_desc * d) {
 //   * head dim 64, several sequences: at most 16 splits, the most that one round of the merge folds (3 x 3096 keys of 2
 //     kv heads 8.20 -> 7.29);
 //   * one round of 8-wave workgroups on the CUs instead of several of 4 waves, whose starts and merges leave the memory
-//     idle: 16 ragged Llama-3-8B caches of 1025 to 8191 keys 61.9 -> 56.8, 4 of 1600 to 6800 22.7 -> 18.4. Launches
-//     that fit two 4-wave workgroups per CU with 128-key splits stay (16 x 396 keys 9.66 against 9.82). Off the
-//     XCD-mapped grid a ragged launch loses a few CUs to uneven dealing, so it is held to 208 workgroups, and splits past
-//     640 keys, where one workgroup too many on a CU costs the most, keep the 4-wave plan (16 Qwen2.5-7B caches of 1.9k
-//     to 10.5k keys: 49.6 us, 58.3 in one round).
+//     idle: 16 ragged Llama-3-8B caches of 1025 to 8191 keys 61.9 -> 56.8, 8 of 1635 to 7245 29.7 -> 28.5. Launches
+//     that fit two 4-wave workgroups per CU with 128-key splits stay (16 x 396 keys 9.66 against 9.82), as do those of
+//     more than 320 MB, whose several rounds overlap (16 caches of 1847 to 8359 keys, 353 MB: 69 against 73). Off the XCD-mapped grid a ragged launch
+//     loses a few CUs to uneven dealing, so it is held to 208 workgroups, and splits past 640 keys, where one workgroup
+//     too many on a CU costs the most, keep the 4-wave plan (16 Qwen2.5-7B caches of 1.9k to 10.5k keys: 49.6 us, 58.3 in
+//     one round).
 struct DecodePlan {
     int64_t chunk;
     int waves;
@@ -153,10 +154,11 @@ struct DecodePlan {
 DecodePlan decode_plan(const mx_attn_desc & d, const int32_t * kv_len, int n_seq, int n_rowtiles, bool xcd) {
     const mx_attn_tuning * t = d.tuning;
     const int64_t quantum = mx::kDecodeChunkQuantum;
-    int64_t lmax = 0, lmin = INT64_MAX;
+    int64_t lmax = 0, lmin = INT64_MAX, keys = 0;
     for (int i = 0; i < n_seq; i++) {
         lmax = std::max<int64_t>(lmax, kv_len[i]);
         lmin = std::min<int64_t>(lmin, kv_len[i]);
+        keys += kv_len[i];
     }
     auto round_up = [&](int64_t x) { return (x + quantum - 1) / quantum * quantum; };
     auto launch_wgs = [&](int64_t c) {
@@ -196,7 +198,7 @@ DecodePlan decode_plan(const mx_attn_desc & d, const int32_t * kv_len, int n_seq
     if (tile && !(xcd && chunk == quantum && launch_wgs(chunk) <= 512)) {
         const bool even = xcd || n_seq == 1;  // every XCD gets the same number of workgroups
         const int64_t c = within(chunk, even ? 256 : 208);
-        if (launch_wgs(c) <= 256 && (even || c <= 640)) return {c, decode_waves(t, c, launch_wgs(c))};
+        if (launch_wgs(c) <= 256 && (even ? keys * d.n_head_kv * d.head_dim * 4 <= ((int64_t)320 << 20) : c <= 640)) return {c, decode_waves(t, c, launch_wgs(c))};
     }
     chunk = within(chunk, workgroup_cap(t));
     return {chunk, decode_waves(t, chunk, launch_wgs(chunk))};
@@ -586,7 +588,6 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
         p.causal = d.causal;
         p.rows = s.rows;
         p.n_rowtiles = s.n_rowtiles;
-        p.seq0 = b0;
         // The XCD-mapped grid (kv head g's splits on XCD g mod 8, partials published into that XCD's L2) for kv heads in
         // multiples of 8, also for batches: Llama-3-8B batch 4 (ragged, 55 MB) 16.97 -> 15.7 us, batch 16 ragged 55.3
         // -> 50.4, 32 x 4096 keys 100.8 -> 97.2 (widened below for short caches)
@@ -604,18 +605,33 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
         const DecodePlan plan = decode_plan(d, kv_len + b0, n_seq, s.n_rowtiles, p.xcd_heads);
         const int64_t chunk = plan.chunk;
         p.chunk = (int32_t)std::min<int64_t>(chunk, INT32_MAX / 2);
+        // the longest sequences first, so that the workgroups past a shorter one's splits come late
+        int order[mx::kMaxSeqPerLaunch];
+        for (int i = 0; i < n_seq; i++) order[i] = b0 + i;
+        std::stable_sort(order, order + n_seq, [&](int x, int y) { return kv_len[x] > kv_len[y]; });
         p.max_split = 1;
-        int32_t xcd0 = 0;
+        p.groups = 0;
         for (int i = 0; i < n_seq; i++) {
-            const int32_t n = kv_len[b0 + i];
-            p.seq[i].k = static_cast<const mx::half_t *>(k_caches[b0 + i]);
-            p.seq[i].v = static_cast<const mx::half_t *>(v_caches[b0 + i]);
+            const int32_t b = order[i], n = kv_len[b];
+            p.seq[i].k = static_cast<const mx::half_t *>(k_caches[b]);
+            p.seq[i].v = static_cast<const mx::half_t *>(v_caches[b]);
             p.seq[i].len = n;
+            p.seq[i].row = b;
             p.seq[i].n_split = (int32_t)((n + p.chunk - 1) / p.chunk);
             p.max_split = std::max(p.max_split, p.seq[i].n_split);
-            p.seq[i].xcd0 = xcd0;
-            xcd0 = (xcd0 + p.seq[i].n_split * d.n_head_kv) % 8;
+            p.seq[i].xcd0 = p.groups % 8;
+            p.first[i] = p.groups;
+            p.groups += p.seq[i].n_split * d.n_head_kv;
         }
+        for (int i = n_seq; i < mx::kMaxSeqPerLaunch; i++) p.first[i] = INT32_MAX;
+        // One round of long 8-wave workgroups on the XCD-mapped grid: a grid of the live groups only. With max_split
+        // splits of every sequence in the grid, the workgroups past a shorter one's splits, though they end at once, upset
+        // the even dealing of the live ones, and one CU too many gets two of those (Llama-3-8B caches in random order, us,
+        // the other grid against this: 8 of 1109 to 8404 keys 51.2 -> 36.8, 12 of 431 to 2177 27.1 -> 18.4, 8 of 588 to
+        // 3507 18.0 -> 18.4). Finding the sequence costs ~0.8 us, so shorter splits keep the other grid (8 of 200 to 1614
+        // keys 10.2 against 10.7).
+        p.flat = n_seq > 1 && p.xcd_heads && plan.waves == 8 && p.chunk >= 384 && p.groups >= 128 &&
+                 p.groups < p.max_split * d.n_head_kv * n_seq;
         for (int i = n_seq; i < mx::kMaxSeqPerLaunch; i++) p.seq[i] = mx::DecodeSeq{};
         // The XCD-mapped grid (partials published into one XCD's L2) also for one short sequence whatever its kv heads:
         // a few splits over at most 4 MB of keys and values, where the merge chain outweighs the stream, which the

@@ -26,7 +26,7 @@ struct DecodeSeq {
     int32_t len;      // keys in the cache
     int32_t n_split;  // splits of `chunk` keys covering them
     int32_t xcd0;     // the XCD of its first workgroup (without xcd_heads): where the sequence before it ended
-    int32_t pad;
+    int32_t row;      // its index in the caller's batch (query and output rows)
 };
 
 struct DecodeParams {
@@ -41,7 +41,6 @@ struct DecodeParams {
     int32_t n_rowtiles;  // ceil(rows / RT)
     int32_t chunk;       // keys per split
     int32_t max_split;   // max over the launch's sequences of n_split
-    int32_t seq0;        // index of the launch's first sequence in the caller's batch (query/output rows)
     int32_t xcd_heads;   // 1: kv head g's splits run on XCD g % 8 (one sequence, n_head_kv a multiple of 8)
     int32_t kv_nt;       // 1: non-temporal K/V loads (one long sequence with xcd_heads, or at least 256 MB of K/V);
                          // honoured by the head-dim-128 kernels with 4-row tiles
@@ -52,6 +51,11 @@ struct DecodeParams {
     float * out32;
     int32_t rope_mode;   // 0 adjacent pairs, 1 split halves (neox), 2 none
     float rope_freq[kMaxHeadDim / 2];  // base^(-2i / head_dim) in f32 for rotary pair i
+    // 1: a 1-D grid of the live (split, kv head) groups only, sequence i's from first[i] on (a batch of sequences with
+    // different split counts); 0: the sequence is blockIdx.y and every one has max_split splits in the grid
+    int32_t flat;
+    int32_t groups;                     // with flat: the groups of all sequences
+    int32_t first[kMaxSeqPerLaunch];    // with flat; past the last sequence INT32_MAX
     DecodeSeq seq[kMaxSeqPerLaunch];
 };
 
@@ -240,7 +244,7 @@ inline size_t linear_counter_bytes(const LinearPlan & l) { return l.splits > 1 ?
 LinearPlan linear_plan(int32_t M, int32_t N, int32_t K, int32_t count, size_t avail);
 hipError_t launch_linear(const LinearParams & p, hipStream_t stream);
 hipError_t launch_stage(const LinearParams & p, hipStream_t stream);  // M > 8: the staged half input rows
-hipError_t launch_gemm(const LinearParams & p, hipStream_t stream);   // M > 8: gemm_kernel on the staged rows
+hipError_t launch_gemm(const LinearParams & p, hipStream_t stream);   // M > 8: the GEMM of p.plan on the staged rows
 hipError_t launch_rope_store(const RopeStoreParams & p, int head_dim, hipStream_t stream);
 hipError_t launch_small_attn(const SmallAttnParams & p, int head_dim, int n_seq, hipStream_t stream);
 // n_batch problems of the prefill kernel along blockIdx.y, offsets from p.*_batch

@@ -325,7 +325,8 @@ def test_workspace_shared_across_shapes(device):
 @pytest.mark.parametrize("H,G,hd", [(4, 4, 64), (20, 20, 64), (14, 2, 64), (32, 8, 128), (12, 4, 128), (4, 1, 256)])
 @pytest.mark.parametrize("lens", [[128], [129], [256, 130, 7], [257, 1], [384, 129, 300, 2], [385, 128], [2049, 300],
                                   [2600] + [100 + 37 * i for i in range(19)], [5000, 4999, 4600, 4200, 4100],
-                                  [1100 - 50 * i for i in range(16)]])
+                                  [1100 - 50 * i for i in range(16)], [1109, 8404, 3000, 5100, 7007, 2222, 6400, 4100],
+                                  [431 + (i * 997) % 1700 for i in range(12)]])
 def test_plan_edges(device, H, G, hd, lens):
     """Lengths at the edges of the split plan (whole sequences, one merge round, one round of 8-wave workgroups, the
     workgroup cap), ragged so that the sequences' workgroups start on different XCDs: f16 and f32 rows against f64."""
