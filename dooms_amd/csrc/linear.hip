@@ -24,8 +24,6 @@
 //   * mx_linear runs these kernels only: no vendor GEMM library is loaded or linked.
 
 #include <algorithm>
-#include <cstdlib>
-#include <cstring>
 #include <type_traits>
 
 #include "mx_common.hpp"
@@ -119,27 +117,8 @@ __global__ __launch_bounds__(kThreads) void stage_kernel(LinearParams p) {
     for (int k = p.K + threadIdx.x * 8; k < kp; k += kThreads * 8) *reinterpret_cast<u32x4 *>(dst + k) = u32x4{0u, 0u, 0u, 0u};
 }
 
-// y (+)= v (+ bias) into row m, column n of output matrix mi.
-template <bool OUT16>
-__device__ __forceinline__ void store_y(const LinearParams & p, int mi, int m, int n, float v) {
-    if (p.flags & kLinearBias) {
-        const float * b = p.bias[mi];
-        if (b) v += b[n];
-    }
-    const int64_t o = (int64_t)m * p.y_stride + n;
-    if constexpr (OUT16) {
-        half_t * y = static_cast<half_t *>(p.y[mi]);
-        if (p.flags & kLinearAccumulate) v += (float)y[o];
-        y[o] = (half_t)v;
-    } else {
-        float * y = static_cast<float *>(p.y[mi]);
-        if (p.flags & kLinearAccumulate) v += y[o];
-        y[o] = v;
-    }
-}
-
 // Epilogue of the tiled GEMMs: the lane's 16 outputs of column n of an MFMA tile (rows mbase + 8 (v / 4) + v % 4),
-// y (+)= acc (+ bias), the same sums as store_y. The bias and the previous outputs are all loaded before the first
+// y (+)= acc (+ bias). The bias and the previous outputs are all loaded before the first
 // store: a store to y may alias them as far as the compiler can tell, so with loads and stores interleaved each
 // element waited for one or two memory round trips in turn. Rows past M read row M - 1 (a valid address) and store
 // nothing.
@@ -366,7 +345,7 @@ __global__ __launch_bounds__(kGemvMaxWaves * kWave) void gemv_kernel(LinearParam
         }
     if (lane < RW * MT) {
         const int i = lane / MT, m = lane % MT, n = r0 + i;
-        if (m < M && n < p.N) {  // store_y's sums, with the bias and the previous output loaded above
+        if (m < M && n < p.N) {  // the bias and the previous output loaded above
             float v = norm ? mine * s_scale[m] : mine;
             if (p.flags & kLinearBias) v += y_bias;
             if (p.flags & kLinearAccumulate) v += y_prev;
