@@ -88,11 +88,10 @@ int32_t hip_status(hipError_t e, const char * what) {
 //     ~5 us more than 32);
 //   * then as small as possible while the launch stays within workgroup_cap() workgroups (measured on MI355X for
 //     Llama-3-8B batches of 4 and 16: 1536 streams best; two workgroups per CU are resident at once, 512 in all).
-// With every split counter on a line of its own (kCounterStride), splitting pays down to the shortest caches: one
-// split per sequence (no merge) no longer wins anywhere measured, e.g. Qwen2.5-0.5B at 513 keys 7.0 us as one split
-// of 8 waves vs 6.5 us as 5 splits of 4 waves, Whisper self-attention at 449 keys 7.1 -> 6.7 us; and 128-key splits
-// beat 256-key ones at every size measured below 32 x 256 keys (Whisper cross-attention over 1500 frames: 7.8 ->
-// 7.25 us, Llama-3-8B at 1024 keys 8.9 -> 8.1 us).
+// With every split counter on a line of its own (kCounterStride), splitting pays from 257 keys (shorter sequences run
+// whole where decode_plan says so): Qwen2.5-0.5B at 513 keys 7.0 us as one split of 8 waves vs 6.5 us as 5 splits of 4
+// waves, Whisper self-attention at 449 keys 7.1 -> 6.7 us; and 128-key splits beat 256-key ones for one sequence below
+// 32 x 256 keys (Whisper cross-attention over 1500 frames: 7.8 -> 7.25 us, Llama-3-8B at 1024 keys 8.9 -> 8.1 us).
 // The bound n_split <= ceil(len / quantum) keeps the workspace a function of the longest sequence alone.
 constexpr int kMaxSplits = 32;
 // One head-dim-128 sequence of at least 32k keys whose 32-split grid would leave CUs idle (fewer than 8 kv heads x row
@@ -132,39 +131,33 @@ DecodeShape decode_shape(const mx_attn_desc * d) {
     return s;
 }
 
-// Keys per split and waves per workgroup of one launch. Besides the plan of the comments above (the shortest splits, then
-// as few as kMaxSplits and the workgroup cap ask for), for one row tile at head dims 64 and 128 (swept over 117 shapes of 1
-// to 16 sequences, f16 and rotated rows; the plan below is within 0.7 % of the best split and waves on average, the
-// plan without it 5.2 %):
-//   * sequences of up to 256 keys (384 at head dim 64) whole, without a merge: 5 x 129 keys of 8 kv heads 6.13 -> 5.31 us,
-//     2 x 163 keys of 20 kv heads 5.25 -> 4.31 with 8 waves; at 388 keys of 20 heads the split is ahead (6.28 against 6.77);
-//   * head dim 64, several sequences: at most 16 splits, the most that one round of the merge folds (3 x 3096 keys of 2
-//     kv heads 8.20 -> 7.29);
-//   * one round of 8-wave workgroups on the CUs instead of several of 4 waves, whose starts and merges leave the memory
-//     idle: 16 ragged Llama-3-8B caches of 1025 to 8191 keys 61.9 -> 56.8, 8 of 1635 to 7245 29.7 -> 28.5. Launches
-//     that fit two 4-wave workgroups per CU with 128-key splits stay (16 x 396 keys 9.66 against 9.82), as do those of
-//     more than 320 MB, whose several rounds overlap (16 caches of 1847 to 8359 keys, 353 MB: 69 against 73). Off the XCD-mapped grid a ragged launch
-//     loses a few CUs to uneven dealing, so it is held to 208 workgroups, and splits past 640 keys, where one workgroup
-//     too many on a CU costs the most, keep the 4-wave plan (16 Qwen2.5-7B caches of 1.9k to 10.5k keys: 49.6 us, 58.3 in
-//     one round).
+// Keys per split and waves per workgroup of one launch: the shortest splits, then as few as kMaxSplits and the workgroup
+// cap ask for (the comments above). For one row tile at head dims 64 and 128 two other plans are taken where they do not
+// lengthen a wave's walk: a wave rounds its probabilities to half against its own running maximum, whose own
+// probability of 1 is exact, so fewer and longer walks round more of them (16 ragged Llama-3-8B caches in one
+// round of 256 workgroups ran 66 -> 63 us, but the output's error against 64 bits went from 2.64e-4 to 2.70e-4):
+//   * sequences of up to 256 keys whole, without a merge, one 32-key block per wave of 8: 8 x 160 keys of 20 kv heads
+//     7.5 -> 6.0 us, 5 x 129 keys of 8 kv heads 6.6 -> 6.1; not f32 rows of head dim 128 with more than 4 rows per kv
+//     head, where the wider tile's merge of 8 waves costs more (256 keys of Qwen2.5-7B 8.2 -> 8.5);
+//   * head dim 64, several sequences: at most 16 splits, the most that one round of the merge folds, with twice the
+//     waves per split (3 x 3096 keys of 2 kv heads 10.8 -> 10.1).
 struct DecodePlan {
     int64_t chunk;
     int waves;
 };
-DecodePlan decode_plan(const mx_attn_desc & d, const int32_t * kv_len, int n_seq, int n_rowtiles, bool xcd) {
+DecodePlan decode_plan(const mx_attn_desc & d, const int32_t * kv_len, int n_seq, const DecodeShape & s, bool f32) {
     const mx_attn_tuning * t = d.tuning;
     const int64_t quantum = mx::kDecodeChunkQuantum;
-    int64_t lmax = 0, lmin = INT64_MAX, keys = 0;
+    int64_t lmax = 0, lmin = INT64_MAX;
     for (int i = 0; i < n_seq; i++) {
         lmax = std::max<int64_t>(lmax, kv_len[i]);
         lmin = std::min<int64_t>(lmin, kv_len[i]);
-        keys += kv_len[i];
     }
     auto round_up = [&](int64_t x) { return (x + quantum - 1) / quantum * quantum; };
     auto launch_wgs = [&](int64_t c) {
         int64_t n = 0;
         for (int i = 0; i < n_seq; i++) n += (kv_len[i] + c - 1) / c;
-        return n * d.n_head_kv * n_rowtiles;
+        return n * d.n_head_kv * s.n_rowtiles;
     };
     // the smallest chunk, at least c, of at most cap workgroups (or the longest sequence whole): bisect over quanta
     auto within = [&](int64_t c, int64_t cap) {
@@ -182,26 +175,28 @@ DecodePlan decode_plan(const mx_attn_desc & d, const int32_t * kv_len, int n_seq
         const int64_t c = round_up((lmax + t->decode_splits - 1) / t->decode_splits);
         return {c, decode_waves(t, c, launch_wgs(c))};
     }
-    const bool tile = n_rowtiles == 1 && (d.head_dim == 64 || d.head_dim == 128) && !(t && t->decode_max_workgroups > 0);
-    const bool hd64 = d.head_dim == 64;
-    if (tile && lmax > quantum && lmax <= (hd64 ? 384 : 256))
-        return {round_up(lmax), t && t->decode_waves ? t->decode_waves : hd64 ? 8 : 4};
-    int64_t msplit = max_splits(&d, n_rowtiles, n_seq, lmax);
-    if (tile && hd64 && n_seq > 1 && lmax <= 16 * 640) msplit = 16;
-    int64_t chunk = round_up((lmax + msplit - 1) / msplit);
-    // A batch of at least 4 sequences of about one length (within 1.5x) and at least 4096 keys: at most 8 splits
-    // per sequence. A/B on one box, us per launch (8 splits of 4 waves against the plan of up to 32): Llama-3-8B
-    // 4 x 8192 keys 29.9 -> 26.4, 8 x 8192 51.9 -> 48.8, 16 x 8192 95.5 -> 90.1, 12 x 4096 42.3 -> 39.9,
-    // Qwen2.5-7B 8 x 4096 22.0 -> 17.7, 4 x 8192 19.5 -> 18.8, Qwen2.5-0.5B 8 x 4096 12.1 -> 9.8. Ragged batches
-    // keep the plan (Qwen2.5-7B 1.3k-7.3k x 16 35 -> 41.7 at 16 splits), as do shorter caches (4 x 2048: 11.5 -> 12.6).
-    if (n_seq >= 4 && lmin >= 4096 && 2 * lmax <= 3 * lmin) chunk = std::max(chunk, round_up((lmax + 7) / 8));
-    if (tile && !(xcd && chunk == quantum && launch_wgs(chunk) <= 512)) {
-        const bool even = xcd || n_seq == 1;  // every XCD gets the same number of workgroups
-        const int64_t c = within(chunk, even ? 256 : 208);
-        if (launch_wgs(c) <= 256 && (even ? keys * d.n_head_kv * d.head_dim * 4 <= ((int64_t)320 << 20) : c <= 640)) return {c, decode_waves(t, c, launch_wgs(c))};
+    // at most msplit splits of the longest sequence
+    auto plan = [&](int64_t msplit) {
+        int64_t chunk = round_up((lmax + msplit - 1) / msplit);
+        // A batch of at least 4 sequences of about one length (within 1.5x) and at least 4096 keys: at most 8 splits
+        // per sequence. A/B on one box, us per launch (8 splits of 4 waves against the plan of up to 32): Llama-3-8B
+        // 4 x 8192 keys 29.9 -> 26.4, 8 x 8192 51.9 -> 48.8, 16 x 8192 95.5 -> 90.1, 12 x 4096 42.3 -> 39.9,
+        // Qwen2.5-7B 8 x 4096 22.0 -> 17.7, 4 x 8192 19.5 -> 18.8, Qwen2.5-0.5B 8 x 4096 12.1 -> 9.8. Ragged batches
+        // keep the plan (Qwen2.5-7B 1.3k-7.3k x 16 35 -> 41.7 at 16 splits), as do shorter caches (4 x 2048: 11.5 ->
+        // 12.6).
+        if (n_seq >= 4 && lmin >= 4096 && 2 * lmax <= 3 * lmin) chunk = std::max(chunk, round_up((lmax + 7) / 8));
+        chunk = within(chunk, workgroup_cap(t));
+        return DecodePlan{chunk, decode_waves(t, chunk, launch_wgs(chunk))};
+    };
+    const DecodePlan base = plan(max_splits(&d, s.n_rowtiles, n_seq, lmax));
+    if (s.n_rowtiles != 1 || (d.head_dim != 64 && d.head_dim != 128) || (t && t->decode_max_workgroups > 0)) return base;
+    if (lmax > quantum && lmax <= 2 * quantum && !(t && t->decode_waves == 4) && (!f32 || d.head_dim == 64 || s.rt == 4))
+        return {2 * quantum, 8};
+    if (d.head_dim == 64 && n_seq > 1 && lmax <= 16 * 640) {
+        const DecodePlan few = plan(16);
+        if (few.chunk * base.waves <= base.chunk * few.waves) return few;  // no more keys per wave
     }
-    chunk = within(chunk, workgroup_cap(t));
-    return {chunk, decode_waves(t, chunk, launch_wgs(chunk))};
+    return base;
 }
 
 // Workspace layout: kMaxTilesPerLaunch split counters (one per (sequence of a launch, kv head, row tile), each on a
@@ -602,7 +597,7 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
         const int64_t kv_bytes = kv_keys * d.kv_stride * 2 * 2;
         p.kv_nt = (p.xcd_heads && kv_bytes >= ((int64_t)16 << 20)) || kv_bytes >= ((int64_t)256 << 20);
         p.scale_log2 = d.scale * 1.4426950408889634f;
-        const DecodePlan plan = decode_plan(d, kv_len + b0, n_seq, s.n_rowtiles, p.xcd_heads);
+        const DecodePlan plan = decode_plan(d, kv_len + b0, n_seq, s, f32);
         const int64_t chunk = plan.chunk;
         p.chunk = (int32_t)std::min<int64_t>(chunk, INT32_MAX / 2);
         // the longest sequences first, so that the workgroups past a shorter one's splits come late
@@ -610,7 +605,7 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
         for (int i = 0; i < n_seq; i++) order[i] = b0 + i;
         std::stable_sort(order, order + n_seq, [&](int x, int y) { return kv_len[x] > kv_len[y]; });
         p.max_split = 1;
-        p.groups = 0;
+        int32_t groups = 0;
         for (int i = 0; i < n_seq; i++) {
             const int32_t b = order[i], n = kv_len[b];
             p.seq[i].k = static_cast<const mx::half_t *>(k_caches[b]);
@@ -619,19 +614,9 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
             p.seq[i].row = b;
             p.seq[i].n_split = (int32_t)((n + p.chunk - 1) / p.chunk);
             p.max_split = std::max(p.max_split, p.seq[i].n_split);
-            p.seq[i].xcd0 = p.groups % 8;
-            p.first[i] = p.groups;
-            p.groups += p.seq[i].n_split * d.n_head_kv;
+            p.seq[i].xcd0 = groups % 8;
+            groups += p.seq[i].n_split * d.n_head_kv;
         }
-        for (int i = n_seq; i < mx::kMaxSeqPerLaunch; i++) p.first[i] = INT32_MAX;
-        // One round of long 8-wave workgroups on the XCD-mapped grid: a grid of the live groups only. With max_split
-        // splits of every sequence in the grid, the workgroups past a shorter one's splits, though they end at once, upset
-        // the even dealing of the live ones, and one CU too many gets two of those (Llama-3-8B caches in random order, us,
-        // the other grid against this: 8 of 1109 to 8404 keys 51.2 -> 36.8, 12 of 431 to 2177 27.1 -> 18.4, 8 of 588 to
-        // 3507 18.0 -> 18.4). Finding the sequence costs ~0.8 us, so shorter splits keep the other grid (8 of 200 to 1614
-        // keys 10.2 against 10.7).
-        p.flat = n_seq > 1 && p.xcd_heads && plan.waves == 8 && p.chunk >= 384 && p.groups >= 128 &&
-                 p.groups < p.max_split * d.n_head_kv * n_seq;
         for (int i = n_seq; i < mx::kMaxSeqPerLaunch; i++) p.seq[i] = mx::DecodeSeq{};
         // The XCD-mapped grid (partials published into one XCD's L2) also for one short sequence whatever its kv heads:
         // a few splits over at most 4 MB of keys and values, where the merge chain outweighs the stream, which the

@@ -259,17 +259,17 @@ void decode_kernel(DecodeParams p) {
     // before the first branch. Otherwise the compiler issues each load after the branch before its first use, and the
     // kernel waits for up to four dependent round trips to the argument memory before its first K/V load. The sequence
     // is blockIdx.y, so its descriptor's address is known at once.
-    int bl = blockIdx.y;
+    const int bl = blockIdx.y;
     const half_t * seq_k = p.seq[bl].k;
     const half_t * seq_v = p.seq[bl].v;
-    int32_t L = p.seq[bl].len, n_split = p.seq[bl].n_split, xcd0 = p.seq[bl].xcd0, flat = p.flat;
+    int32_t L = p.seq[bl].len, n_split = p.seq[bl].n_split, xcd0 = p.seq[bl].xcd0;
     uint32_t T = p.n_rowtiles;
     int32_t max_split = p.max_split, n_head_kv = p.n_head_kv, chunk = p.chunk, G = p.group, seq0 = p.seq[bl].row, n_q = p.n_q;
     int32_t rows = p.rows, causal = p.causal, xcd_heads = p.xcd_heads;
     int64_t q_stride = p.q_stride, kv_stride = p.kv_stride;
     const half_t * qp = p.q;
-    asm volatile("" : "+s"(seq_k), "+s"(seq_v), "+s"(L), "+s"(n_split), "+s"(xcd0), "+s"(flat), "+s"(T), "+s"(max_split), "+s"(n_head_kv),
-                 "+s"(chunk), "+s"(G), "+s"(seq0), "+s"(n_q), "+s"(rows), "+s"(causal), "+s"(xcd_heads), "+s"(q_stride),
+    asm volatile("" : "+s"(seq_k), "+s"(seq_v), "+s"(L), "+s"(n_split), "+s"(xcd0), "+s"(T), "+s"(max_split),
+                 "+s"(n_head_kv), "+s"(chunk), "+s"(G), "+s"(seq0), "+s"(n_q), "+s"(rows), "+s"(causal), "+s"(xcd_heads), "+s"(q_stride),
                  "+s"(kv_stride), "+s"(qp));
     // the fused step's own arguments likewise (fetched behind branches they cost dependent scalar round trips ahead
     // of the first K/V load)
@@ -298,29 +298,14 @@ void decode_kernel(DecodeParams p) {
     const uint32_t id = blockIdx.x, k8 = id / 8, u = k8 / T;
     const int rt = k8 % T;
     int s, g;  // split, kv head
-    uint32_t grp = u * 8 + id % 8;  // (split, kv head) group: of the sequence, or of the launch
-    if (flat) {
-        // the live groups of a ragged batch, sequence after sequence: the one that holds this group by a scan of their
-        // first groups, then its descriptor (dependent scalar loads, ~0.8 us, which only these launches pay)
-        if (grp >= (uint32_t)p.groups) return;  // padding of the grid to whole XCD rounds
-#pragma unroll
-        for (int i = 1; i < kMaxSeqPerLaunch; i++) bl += grp >= (uint32_t)p.first[i] ? 1 : 0;
-        grp -= (uint32_t)p.first[bl];
-        seq_k = p.seq[bl].k;
-        seq_v = p.seq[bl].v;
-        L = p.seq[bl].len;
-        n_split = p.seq[bl].n_split;
-        seq0 = p.seq[bl].row;
-        max_split = n_split;
-    }
     if (xcd_heads) {
-        const uint32_t v = grp / 8;
-        s = v % max_split;
-        g = (v / max_split) * 8 + grp % 8;
+        s = u % max_split;
+        g = (u / max_split) * 8 + id % 8;
     } else {
-        // the sequence's first group on the XCD after the previous sequence's last: the live workgroups of a ragged batch
-        // spread evenly over the XCDs (numbered by the longest sequence's splits, those of shorter ones fell on a few)
-        if (!flat) grp = u * 8 + (id - (uint32_t)xcd0) % 8;
+        // (split, kv head) group of the sequence, the first on the XCD after the previous sequence's last: the live
+        // workgroups of a ragged batch spread evenly over the XCDs (numbered by the longest sequence's splits, those of
+        // shorter ones fell on a few)
+        const uint32_t grp = u * 8 + (id - (uint32_t)xcd0) % 8;
         s = grp % n_split;
         g = grp / n_split;
     }
@@ -788,8 +773,8 @@ template <int HD, int RT, int NW>
 hipError_t launch_decode_t(const DecodeParams & p, int n_seq, hipStream_t stream) {
     // x: groups of (split, kv head), 8 per round of XCDs, each group's row tiles on one XCD; y: the sequence
     // (the XCD-mapped grid: kv head g's splits at ids = g mod 8, so the kv heads round up to a multiple of 8)
-    const int64_t groups = p.flat ? p.groups : (int64_t)p.max_split * (p.xcd_heads ? (p.n_head_kv + 7) / 8 * 8 : p.n_head_kv);
-    const dim3 grid((uint32_t)(((groups + 7) / 8) * 8 * p.n_rowtiles), p.flat ? 1u : (uint32_t)n_seq);
+    const int64_t groups = (int64_t)p.max_split * (p.xcd_heads ? (p.n_head_kv + 7) / 8 * 8 : p.n_head_kv);
+    const dim3 grid((uint32_t)(((groups + 7) / 8) * 8 * p.n_rowtiles), (uint32_t)n_seq);
     if constexpr (HD == 128 && RT == 4) {  // one query row per Llama-3-8B-shaped sequence (4 query heads per kv head)
         if (p.kv_nt) {
             if (p.f32)

@@ -41,7 +41,7 @@ struct DecodeParams {
     int32_t n_rowtiles;  // ceil(rows / RT)
     int32_t chunk;       // keys per split
     int32_t max_split;   // max over the launch's sequences of n_split
-    int32_t xcd_heads;   // 1: kv head g's splits run on XCD g % 8 (one sequence, n_head_kv a multiple of 8)
+    int32_t xcd_heads;   // 1: kv head g's splits run on XCD g % 8 (n_head_kv a multiple of 8, or one short sequence)
     int32_t kv_nt;       // 1: non-temporal K/V loads (one long sequence with xcd_heads, or at least 256 MB of K/V);
                          // honoured by the head-dim-128 kernels with 4-row tiles
     float scale_log2;    // scale * log2(e): scores are kept in base-2 units
@@ -51,11 +51,6 @@ struct DecodeParams {
     float * out32;
     int32_t rope_mode;   // 0 adjacent pairs, 1 split halves (neox), 2 none
     float rope_freq[kMaxHeadDim / 2];  // base^(-2i / head_dim) in f32 for rotary pair i
-    // 1: a 1-D grid of the live (split, kv head) groups only, sequence i's from first[i] on (a batch of sequences with
-    // different split counts); 0: the sequence is blockIdx.y and every one has max_split splits in the grid
-    int32_t flat;
-    int32_t groups;                     // with flat: the groups of all sequences
-    int32_t first[kMaxSeqPerLaunch];    // with flat; past the last sequence INT32_MAX
     DecodeSeq seq[kMaxSeqPerLaunch];
 };
 
