@@ -400,6 +400,18 @@ def test_stream_k_partition(tmp_path):
     assert "0 failures" in r.stdout
 
 
+def test_decode_plan(tmp_path):
+    # the decode kernel's split plan (api.hip: decode_plan), by tests/cpp/decode_plan_check.cpp, which includes the source;
+    # the launches it names are never called
+    exe = tmp_path / "decode_plan_check"
+    src = os.path.join(ROOT, "tests", "cpp", "decode_plan_check.cpp")
+    subprocess.run(["/opt/rocm/bin/hipcc", "-O1", "-std=c++17", "--offload-arch=gfx950", "-Wno-unused-function",
+                    "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "dooms_amd", "csrc"), src,
+                    "-Wl,--unresolved-symbols=ignore-all", "-Wl,-z,lazy", "-o", str(exe)], check=True, capture_output=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+
+
 def test_gemm_load_rows(tmp_path):
     # the rows the 128 x 128 GEMM's loads read (mx_kernels.hpp: gemm_load_row), by tests/cpp/gemm_rows_check.cpp
     exe = tmp_path / "gemm_rows_check"
