@@ -140,7 +140,8 @@ DecodeShape decode_shape(const mx_attn_desc * d) {
 //     7.5 -> 6.0 us, 5 x 129 keys of 8 kv heads 6.6 -> 6.1; not f32 rows of head dim 128 with more than 4 rows per kv
 //     head, where the wider tile's merge of 8 waves costs more (256 keys of Qwen2.5-7B 8.2 -> 8.5), nor f32 rows of head
 //     dim 64 past one workgroup per CU, which is what their registers allow (12 x 130 keys of 20 kv heads 7.0 split,
-//     8.1 whole; f16 rows fit two and stay ahead: 16 x 140 keys 7.6 -> 6.4);
+//     8.1 whole; f16 rows fit two and stay ahead: 16 x 140 keys 7.6 -> 6.4), nor where the workgroup cap leaves the
+//     sequences whole anyway, on 4 waves (32 x 140 keys of 28 kv heads, f16, 10.6 on 4 waves, 12.1 on 8);
 //   * head dim 64, several sequences: at most 16 splits, the most that one round of the merge folds, with twice the
 //     waves per split (3 x 3096 keys of 2 kv heads 10.8 -> 10.1).
 struct DecodePlan {
@@ -193,7 +194,8 @@ DecodePlan decode_plan(const mx_attn_desc & d, const int32_t * kv_len, int n_seq
     const DecodePlan base = plan(max_splits(&d, s.n_rowtiles, n_seq, lmax));
     if (s.n_rowtiles != 1 || (d.head_dim != 64 && d.head_dim != 128) || (t && t->decode_max_workgroups > 0)) return base;
     const bool fits = !f32 || (d.head_dim == 64 ? launch_wgs(2 * quantum) <= 256 : s.rt == 4);
-    if (lmax > quantum && lmax <= 2 * quantum && !(t && t->decode_waves == 4) && fits) return {2 * quantum, 8};
+    if (lmax > quantum && base.chunk == quantum && lmax <= 2 * quantum && !(t && t->decode_waves == 4) && fits)
+        return {2 * quantum, 8};
     if (d.head_dim == 64 && n_seq > 1 && lmax <= 16 * 640) {
         const DecodePlan few = plan(16);
         if (few.chunk * base.waves <= base.chunk * few.waves) return few;  // no more keys per wave
