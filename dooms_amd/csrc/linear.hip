@@ -558,8 +558,8 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     }
     auto issue = [&](int step, int buf) __attribute__((always_inline)) {
         const int64_t k0 = (int64_t)(s0 + step) * BK * 2;
-        // the last step of a K that is an odd multiple of 32: the staged rows are zero-padded, the weights' chunks past
-        // the row read the four before them (finite values that meet the zeros)
+        // the last step of a K that is an odd multiple of 32: the chunks past the weights' row read the four before them,
+        // and the products of the columns past K are left out (zeros of the staged rows would make NaN of an infinity)
         const bool half_step = BK == 64 && (s0 + step) * BK + BK > p.K;
 #pragma unroll
         for (int i = 0; i < LPS; i++) {
@@ -585,6 +585,7 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
         if (a < nk) issue(a, a);
     for (int s = 0; s < nk; s++) {
         const int buf = s % NBUF;
+        const bool half_step = BK == 64 && (s0 + s) * BK + BK > p.K;
         const int later = min(NBUF - 2, nk - 1 - s);
         static_for<0, NBUF - 1>([&](auto R) __attribute__((always_inline)) {
             constexpr int n = decltype(R)::value * LPS;
@@ -617,10 +618,12 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
             if constexpr (ks + 1 < KS) asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(MI + NJ) : "memory");
             else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_sched_barrier(0);
+            if (BK == 128 || ks == 0 || !half_step) {
 #pragma unroll
-            for (int i = 0; i < MI; i++)
+                for (int i = 0; i < MI; i++)
 #pragma unroll
-                for (int j = 0; j < NJ; j++) acc[i][j] = mfma16x16x32(as_half8(fw[ks][j]), as_half8(fx[ks][i]), acc[i][j]);
+                    for (int j = 0; j < NJ; j++) acc[i][j] = mfma16x16x32(as_half8(fw[ks][j]), as_half8(fx[ks][i]), acc[i][j]);
+            }
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (ks + 2 < KS) reads(std::integral_constant<int, ks + 2>{});
         });

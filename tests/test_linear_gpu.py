@@ -147,6 +147,27 @@ def test_gemm_parts_of_k(device, M, N, K, opts):
     run(device, 80 + M + K, M, N, K, **opts)
 
 
+@pytest.mark.parametrize("M,N,K", [(24, 136, 96), (150, 200, 160), (300, 520, 1056), (1024, 4096, 2080)])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_gemm_infinite_weights_beside_the_padding(device, M, N, K, value):
+    """K an odd multiple of 32: the last step's columns past K hold no product, so an infinite weight anywhere in the row
+    gives the infinity (positive inputs), a NaN a NaN, and no other column changes."""
+    assert K % 64 == 32
+    rng = np.random.default_rng(K)
+    x = torch.from_numpy(rng.uniform(0.5, 2, (M, K)).astype(np.float32)).to(device)
+    w = torch.from_numpy((rng.standard_normal((N, K), dtype=np.float32) / np.sqrt(K)).astype(np.float16)).to(device)
+    ref = A.linear(x, w)
+    cols = list(range(K - 40, K)) + [0, K // 2]
+    for i, k in enumerate(cols):
+        w[3 * i, k] = value
+    out = A.linear(x, w)
+    hit = torch.zeros(N, dtype=torch.bool, device=device)
+    hit[[3 * i for i in range(len(cols))]] = True
+    assert torch.equal(out[:, ~hit], ref[:, ~hit])
+    got = out[:, hit]
+    assert bool((got.isnan() if np.isnan(value) else got == value).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(24, 256, 4096), (200, 320, 1280)])
 def test_gemm_workspace_of_the_staged_rows_alone(device, M, N, K):
     """A workspace with room for the staged rows only (and for a part of what the plan would take) still runs, with
