@@ -18,6 +18,7 @@
 #include <queue>
 #include <string>
 
+#include "linear_plan.hpp"
 #include "mx_kernels.hpp"
 
 namespace {

@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "linear_plan.hpp"
 #include "mx_common.hpp"
 #include "mx_kernels.hpp"
 
@@ -371,11 +372,14 @@ __global__ __launch_bounds__(kGemvMaxWaves * kWave) void gemv_kernel(LinearParam
 // 14336 445 -> 392. The raised wave priority around the products, the loads all in the first phase, spread over all
 // four or ahead of the operand reads, and phases of two slices measured 1 to 10 % slower.
 // BN = 192 (256 x 192, 8 waves of 64 x 96) serves products whose 256 x 256 tiles would leave CUs idle.
-constexpr int kBM = 256;
-constexpr int kGemmCUs = 256;
+constexpr int kBM = kGemmBigRows;
 constexpr int kBigWaves = 8, kBigThreads = kBigWaves * kWave;
 // WC: columns per wave (64, or 96 for 256 x 192 tiles: 8 waves of 64 x 96).
-template <bool OUT16, int BN, int WC>
+// HALF: K is an odd multiple of 32. The staged rows are zero-padded to the last step's 64 columns, the chunks past the
+// weights' row read the four before them, and the last step's second half takes no part in the products (zeros of the
+// staged rows would make NaN of an infinity). Walked in 32-column steps through three buffers, 2048 x 6144 x 4128 took
+// 131 us, on 128-row tiles 138, so 117 (3000 x 4096 x 14304 445, 501 and 426).
+template <bool OUT16, int BN, int WC, bool HALF>
 __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
     constexpr int kBN = BN, kBK = 64;
     constexpr int kBlocks = (kBM + BN) / 8;                  // 1 KB blocks (8 rows x 128 bytes) of a step's tiles
@@ -392,25 +396,30 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
     const int l32 = lane % 32, hi = lane / 32;
 
-    // Each lane's source bytes relative to the step's first column are fixed: rows past M (N) repeat the last row.
-    // K is a multiple of 64 here, so the staged rows are K halves apart, as the weight rows. Lane l of block j fills
-    // position l % 8 of the tile's row 8 j + l / 8 with 16-byte chunk (l % 8) ^ (row / 2 % 8).
-    const char * a_base = reinterpret_cast<const char *>(p.xh + (int64_t)m0 * p.K);
+    // Each lane's source bytes relative to the step's first column are fixed: rows past M (N) repeat the last row. The
+    // staged rows are K rounded up to 64 halves apart. Lane l of block j fills position l % 8 of the tile's row
+    // 8 j + l / 8 with 16-byte chunk (l % 8) ^ (row / 2 % 8).
+    const int kp = HALF ? p.K + 32 : p.K, nk = kp / kBK;
+    const char * a_base = reinterpret_cast<const char *>(p.xh + (int64_t)m0 * kp);
     const char * b_base = reinterpret_cast<const char *>(p.w[mi] + (int64_t)n0 * p.K);
     uint32_t off[Loads];
 #pragma unroll
     for (int i = 0; i < Loads; i++) {
         const int row = 8 * (i * kBigWaves + wave) + lane / 8;
         const int r = row < kBM ? gemm_load_row(m0, row, p.M) - m0 : gemm_load_row(n0, row - kBM, p.N) - n0;
-        off[i] = (uint32_t)r * (uint32_t)p.K * 2 + 16 * ((lane % 8) ^ ((row >> 1) & 7));
+        off[i] = (uint32_t)r * (uint32_t)(row < kBM ? kp : p.K) * 2 + 16 * ((lane % 8) ^ ((row >> 1) & 7));
     }
+    // HALF: what this lane's weight loads of the last step go back (its chunk is the same for all of them)
+    const uint32_t back = HALF && ((lane % 8) ^ ((4 * wave + lane / 16) & 7)) >= 4 ? 64 : 0;
     // loads I0 .. I1 - 1 of a step
     auto issue = [&](int step, auto I0C, auto I1C) __attribute__((always_inline)) {
         const int64_t k0 = (int64_t)step * kBK * 2;  // bytes
         static_for<decltype(I0C)::value, decltype(I1C)::value>([&](auto I) __attribute__((always_inline)) {
             constexpr int i = decltype(I)::value;
+            constexpr bool a = i * kBigWaves < kBM / 8;
             const int j = i * kBigWaves + wave;
-            __builtin_amdgcn_global_load_lds((i * kBigWaves < kBM / 8 ? a_base : b_base) + k0 + off[i],
+            const uint32_t o = HALF && !a && step == nk - 1 ? off[i] - back : off[i];
+            __builtin_amdgcn_global_load_lds((a ? a_base : b_base) + k0 + o,
                                              (__attribute__((address_space(3))) void *)&sm[step & 1][512 * j], 16, 0, 0);
         });
     };
@@ -438,7 +447,6 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("" ::: "memory");
     };
-    const int nk = p.K / kBK;
     using I0 = std::integral_constant<int, 0>;
     using IH = std::integral_constant<int, Loads / 2>;
     using IE = std::integral_constant<int, Loads>;
@@ -481,12 +489,12 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
                 if (behind) __builtin_amdgcn_s_waitcnt(0x0F70);
             }
             barrier();
-            
+            if (!HALF || ks < 2 || s + 1 < nk) {
 #pragma unroll
-            for (int i = 0; i < kBigMI; i++)
+                for (int i = 0; i < kBigMI; i++)
 #pragma unroll
-                for (int j = 0; j < kBigNJ; j++) acc[i][j] = mfma32x32x16(as_half8(fa[i]), as_half8(fb[j]), acc[i][j]);
-            
+                    for (int j = 0; j < kBigNJ; j++) acc[i][j] = mfma32x32x16(as_half8(fa[i]), as_half8(fb[j]), acc[i][j]);
+            }
             if constexpr (ks == 3) {
                 if (!behind) __builtin_amdgcn_s_waitcnt(0x0F70);
             }
@@ -505,10 +513,10 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
         }
 }
 
-template <bool OUT16>
-__global__ __launch_bounds__(kBigThreads, 1) void gemm_big_kernel(LinearParams p) { gemm_big_tile<OUT16, 256, 64>(p); }
-template <bool OUT16>
-__global__ __launch_bounds__(kBigThreads, 1) void gemm_w192_kernel(LinearParams p) { gemm_big_tile<OUT16, 192, 96>(p); }
+template <bool OUT16, bool HALF>
+__global__ __launch_bounds__(kBigThreads, 1) void gemm_big_kernel(LinearParams p) { gemm_big_tile<OUT16, 256, 64, HALF>(p); }
+template <bool OUT16, bool HALF>
+__global__ __launch_bounds__(kBigThreads, 1) void gemm_w192_kernel(LinearParams p) { gemm_big_tile<OUT16, 192, 96, HALF>(p); }
 
 // ---- M > 8, products with too few 256-row tiles for the chip: BM x BN tiles of 4 waves, K cut into p.plan.splits parts ----
 // Few rows are bound by the weights' stream from HBM (24 x 4096 x 4096: 33.5 MB, 5.2 us at 6.4 TB/s), which needs every
@@ -518,7 +526,8 @@ __global__ __launch_bounds__(kBigThreads, 1) void gemm_w192_kernel(LinearParams 
 // tile lies whole in LDS with its 16-byte chunks permuted by the row (chunk ^ r % 16, or ^ r / 2 % 8 with 128-byte rows): the
 // 16-byte operand reads of 16 rows at one chunk hit 16 distinct 4-bank groups. The weights are MFMA operand A, so that
 // a lane holds 4 consecutive outputs of one row (16-byte stores).
-template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF>
+// HALF: K is an odd multiple of 32, as in gemm_big_tile; the last part's last step is half padding.
+template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF, bool HALF>
 __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     constexpr int WN = kWaves / WM;                        // waves along the weight rows
     constexpr int MI = BM / WM / 16, NJ = BN / WN / 16;    // 16 x 16 MFMA tiles per wave
@@ -526,6 +535,7 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     constexpr int XB = BM / RPB, WB = BN / RPB;            // load blocks of a step
     constexpr int LPS = (XB + WB) / kWaves;                // loads per wave and step
     constexpr int KS = BK / 32;                            // MFMA steps per K step
+    static_assert(!HALF || BK == 64, "a last step of 32 columns and 32 of padding");
     static_assert((XB + WB) % kWaves == 0 && MI >= 1 && NJ >= 1 && LPS * (NBUF - 1) < 64, "whole loads and tiles");
     __shared__ __attribute__((aligned(1024))) half_t sm[NBUF][(BM + BN) * BK];
     __shared__ int s_last;
@@ -539,8 +549,8 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     const int tile = (mi * n_tiles + nt) * m_tiles + mt;
     const int m0 = mt * BM, n0 = nt * BN;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
-    const int kp = (p.K + 63) / 64 * 64;
-    const int steps = BK == 64 ? kp / 64 : p.K / BK, s0 = (int)((int64_t)split * steps / S), nk = (int)((int64_t)(split + 1) * steps / S) - s0;
+    const int kp = HALF ? p.K + 32 : p.K;
+    const int steps = kp / BK, s0 = (int)((int64_t)split * steps / S), nk = (int)((int64_t)(split + 1) * steps / S) - s0;
 
     // load block j = i kWaves + wave of a step: RPB rows x BK columns; lane l fills position l % CH of row l / CH with
     // chunk (l % CH) ^ swizzle(row)
@@ -558,15 +568,13 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     }
     auto issue = [&](int step, int buf) __attribute__((always_inline)) {
         const int64_t k0 = (int64_t)(s0 + step) * BK * 2;
-        // the last step of a K that is an odd multiple of 32: the chunks past the weights' row read the four before them,
-        // and the products of the columns past K are left out (zeros of the staged rows would make NaN of an infinity)
-        const bool half_step = BK == 64 && (s0 + step) * BK + BK > p.K;
+        const bool half_step = HALF && (s0 + step) * BK + BK > p.K;
 #pragma unroll
         for (int i = 0; i < LPS; i++) {
             const int j = i * kWaves + wave;
             const char * src = (j < XB ? xg : wg) + k0;
             uint32_t o = off[i];
-            if (BK == 64 && __builtin_expect(half_step, 0) && j >= XB && ((lane % CH) ^ swz((j - XB) * RPB + lane / CH)) >= 4) o -= 64;
+            if (half_step && j >= XB && ((lane % CH) ^ swz((j - XB) * RPB + lane / CH)) >= 4) o -= 64;
             __builtin_amdgcn_global_load_lds(src + o, (__attribute__((address_space(3))) void *)&sm[buf][512 * j], 16, 0, 0);
         }
     };
@@ -585,7 +593,7 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
         if (a < nk) issue(a, a);
     for (int s = 0; s < nk; s++) {
         const int buf = s % NBUF;
-        const bool half_step = BK == 64 && (s0 + s) * BK + BK > p.K;
+        const bool half_step = HALF && (s0 + s) * BK + BK > p.K;
         const int later = min(NBUF - 2, nk - 1 - s);
         static_for<0, NBUF - 1>([&](auto R) __attribute__((always_inline)) {
             constexpr int n = decltype(R)::value * LPS;
@@ -618,7 +626,7 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
             if constexpr (ks + 1 < KS) asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(MI + NJ) : "memory");
             else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_sched_barrier(0);
-            if (BK == 128 || ks == 0 || !half_step) {
+            if (!HALF || ks == 0 || !half_step) {
 #pragma unroll
                 for (int i = 0; i < MI; i++)
 #pragma unroll
@@ -742,42 +750,42 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     }
 }
 
-template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF>
-__global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(LinearParams p) { gemm_split_tile<OUT16, BM, BN, WM, BK, NBUF>(p); }
+template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF, bool HALF>
+__global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(LinearParams p) { gemm_split_tile<OUT16, BM, BN, WM, BK, NBUF, HALF>(p); }
 
-// The GEMM's tile shapes and what a product costs on each, in microseconds, fitted (least relative squares, 8 % rms) to
-// 4700 measured launches: 9 to 4096 rows of the decoders' projections, every shape with 1 to 12 parts of K.
-//   t = 4.5 + 0.2 M K / 1e6 (staging) + 1.06 M N / 1e6 (output)                       the same for every shape
-//     + rounds * (tile + steps * step)     steps of 64 columns per part; a round is one workgroup per CU, or two where
-//                                          per_cu is 2 (a part round of at most one per CU takes step1, else step2)
-//     + (parts > 1) * (merge * (1 + parts * tile bytes / 64 KB) + part_mb * partial MB)
-// Picking the cheapest is within 1.1 % of the measured best on average over those products (the worst 19 %). What the
-// split buys, against the 128 x 128 tiles with whole K that took every product of few tiles (us, staging included):
-// 24 x 4096 x 4096 47.9 -> 12.9, 64 x 4096 x 4096 49.0 -> 15.3, 256 x 4096 x 4096 51.0 -> 24.6, 24 x 4096 x 14336
-// 147 -> 29.4, 512 x 1152 x 896 19.1 -> 10.0, 1024 x 3584 x 3584 50.2 -> 46.
-struct GemmCfg {
-    int bm, bn, bk, threads, per_cu;
-    float step1, step2, tile, merge, part_mb;
+// The kernels of kGemmCfgs, by shape: f32 and f16 outputs, and those of a K that is an odd multiple of 32, for the shapes
+// that take one.
+struct GemmKernels {
+    int threads;
     void (*k32)(LinearParams);
     void (*k16)(LinearParams);
+    void (*half32)(LinearParams);
+    void (*half16)(LinearParams);
 };
-constexpr int kGemmCfgs = 8;
-constexpr int kMaxParts = 12, kMaxSplitGrid = 1024;  // the fitted range
-const GemmCfg & gemm_cfg(int c) {
-#define MX_SPLIT(BM, BN, WM, BK, NB, CU, ...) \
-    {BM, BN, BK, kThreads, CU, __VA_ARGS__, gemm_split_kernel<false, BM, BN, WM, BK, NB>, gemm_split_kernel<true, BM, BN, WM, BK, NB>}
-    static const GemmCfg cfgs[kGemmCfgs] = {
-        MX_SPLIT(16, 64, 1, 128, 6, 1, 0.219f, 0.f, 0.315f, 0.539f, 1.588f),
-        MX_SPLIT(32, 64, 1, 128, 3, 2, 0.250f, 0.402f, 0.f, 0.899f, 0.522f),
-        MX_SPLIT(64, 64, 2, 64, 4, 2, 0.340f, 0.553f, 0.f, 0.920f, 0.415f),
-        MX_SPLIT(128, 64, 2, 128, 3, 1, 0.421f, 0.f, 1.094f, 0.765f, 0.348f),
-        MX_SPLIT(128, 128, 2, 64, 4, 1, 0.640f, 0.f, 2.207f, 0.930f, 0.203f),
-        MX_SPLIT(128, 128, 2, 64, 2, 2, 0.887f, 1.078f, 0.f, 1.092f, 0.306f),
-        {256, 192, 64, kBigThreads, 1, 1.243f, 0.f, 5.946f, 0.f, 0.f, gemm_w192_kernel<false>, gemm_w192_kernel<true>},
-        {256, 256, 64, kBigThreads, 1, 1.426f, 0.f, 8.941f, 0.f, 0.f, gemm_big_kernel<false>, gemm_big_kernel<true>},
+template <int BM, int BN, int WM, int BK, int NBUF>
+constexpr GemmKernels split_kernels() {
+    GemmKernels k{kThreads, gemm_split_kernel<false, BM, BN, WM, BK, NBUF, false>, gemm_split_kernel<true, BM, BN, WM, BK, NBUF, false>,
+                  nullptr, nullptr};
+    if constexpr (BK == 64) {
+        k.half32 = gemm_split_kernel<false, BM, BN, WM, BK, NBUF, true>;
+        k.half16 = gemm_split_kernel<true, BM, BN, WM, BK, NBUF, true>;
+    }
+    return k;
+}
+const GemmKernels & gemm_kernels(int cfg) {
+    static const GemmKernels kernels[kNumGemmCfgs] = {
+        split_kernels<16, 64, 1, 128, 6>(),
+        split_kernels<32, 64, 1, 128, 3>(),
+        split_kernels<64, 64, 2, 64, 4>(),
+        split_kernels<128, 64, 2, 128, 3>(),
+        split_kernels<128, 128, 2, 64, 4>(),
+        split_kernels<128, 128, 2, 64, 2>(),
+        {kBigThreads, gemm_w192_kernel<false, false>, gemm_w192_kernel<true, false>, gemm_w192_kernel<false, true>,
+         gemm_w192_kernel<true, true>},
+        {kBigThreads, gemm_big_kernel<false, false>, gemm_big_kernel<true, false>, gemm_big_kernel<false, true>,
+         gemm_big_kernel<true, true>},
     };
-#undef MX_SPLIT
-    return cfgs[c];
+    return kernels[cfg];
 }
 
 // Waves per workgroup: the (matrix, RW-row group) items spread evenly over the CUs, one workgroup per CU (the weight
@@ -835,40 +843,11 @@ hipError_t launch_linear(const LinearParams & p, hipStream_t stream) {
     return launch_gemm(p, stream);
 }
 
-LinearPlan linear_plan(int32_t M, int32_t N, int32_t K, int32_t count, size_t avail) {
-    LinearPlan best{-1, 1, 0, 0};
-    float best_t = 0.f;
-    for (int i = 0; i < kGemmCfgs; i++) {
-        const GemmCfg & c = gemm_cfg(i);
-        // the split GEMM's 64-column shapes take any K (a multiple of 32), so that some shape always applies
-        if (K % (c.bk == 128 ? 128 : c.bm == kBM ? 64 : 32)) continue;
-        const int64_t tiles = (int64_t)count * ((N + c.bn - 1) / c.bn) * ((M + c.bm - 1) / c.bm);
-        const int ksteps = (K + c.bk - 1) / c.bk;
-        const int most = c.merge > 0.f ? (int)std::min<int64_t>(std::min(kMaxParts, ksteps), kMaxSplitGrid / tiles) : 1;
-        for (int s = 1; s <= std::max(most, 1); s++) {
-            const LinearPlan l{i, s, (int32_t)tiles, 0};
-            const size_t part_bytes = s > 1 ? (size_t)tiles * s * c.bm * c.bn * 4 : 0;
-            const size_t bytes = part_bytes + linear_counter_bytes(l);
-            if (bytes > avail) break;
-            const int64_t wgs = tiles * s, slots = (int64_t)kGemmCUs * c.per_cu, full = wgs / slots, rem = wgs % slots;
-            const float steps = (float)((ksteps + s - 1) / s) * (float)(c.bk / 64);
-            const float n1 = (float)((c.per_cu == 1 ? full : 0) + (rem > 0 && rem <= kGemmCUs ? 1 : 0));
-            const float n2 = (float)((c.per_cu == 1 ? 0 : full) + (rem > kGemmCUs ? 1 : 0));
-            float t = (n1 + n2) * c.tile + steps * (n1 * c.step1 + n2 * c.step2);
-            if (s > 1) t += c.merge * (1.f + (float)(s * c.bm * c.bn * 4) / 65536.f) + c.part_mb * (float)part_bytes * 1e-6f;
-            if (best.cfg < 0 || t < best_t) {
-                best = l;
-                best.bytes = bytes;
-                best_t = t;
-            }
-        }
-    }
-    return best;
-}
-
 hipError_t launch_gemm(const LinearParams & p, hipStream_t stream) {
-    const GemmCfg & c = gemm_cfg(p.plan.cfg);
-    hipLaunchKernelGGL((p.flags & kLinearOutF16) ? c.k16 : c.k32, dim3((uint32_t)(p.plan.tiles * p.plan.splits)), dim3(c.threads), 0, stream, p);
+    const GemmKernels & k = gemm_kernels(p.plan.cfg);
+    const bool out16 = p.flags & kLinearOutF16, half = p.K % 64 != 0;
+    hipLaunchKernelGGL(half ? (out16 ? k.half16 : k.half32) : (out16 ? k.k16 : k.k32), dim3((uint32_t)(p.plan.tiles * p.plan.splits)),
+                       dim3(k.threads), 0, stream, p);
     return hipGetLastError();
 }
 

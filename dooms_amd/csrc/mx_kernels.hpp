@@ -233,10 +233,6 @@ hipError_t launch_fill_zero(void * p, size_t bytes, hipStream_t stream);
 // query rows one prefill workgroup covers (forced: a plan fixed by the caller, or 0)
 int prefill_rows_per_workgroup(int n_q, int n_head, int n_kv, int head_dim, int forced);
 hipError_t launch_prefill(const PrefillParams & p, int head_dim, hipStream_t stream);
-// counters of a split GEMM, each on a 256-byte line of its own
-inline size_t linear_counter_bytes(const LinearPlan & l) { return l.splits > 1 ? (size_t)l.tiles * kCounterStride * 4 : 0; }
-// avail: workspace bytes behind the staged rows that the plan may use
-LinearPlan linear_plan(int32_t M, int32_t N, int32_t K, int32_t count, size_t avail);
 hipError_t launch_linear(const LinearParams & p, hipStream_t stream);
 hipError_t launch_stage(const LinearParams & p, hipStream_t stream);  // M > 8: the staged half input rows
 hipError_t launch_gemm(const LinearParams & p, hipStream_t stream);   // M > 8: the GEMM of p.plan on the staged rows

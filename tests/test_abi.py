@@ -412,6 +412,18 @@ def test_decode_plan(tmp_path):
     assert r.returncode == 0, r.stdout
 
 
+def test_linear_plan(tmp_path):
+    # the projections' plan (linear_plan.hpp), by tests/cpp/linear_plan_check.cpp
+    exe = tmp_path / "linear_plan_check"
+    src = os.path.join(ROOT, "tests", "cpp", "linear_plan_check.cpp")
+    subprocess.run(["/opt/rocm/bin/hipcc", "-O2", "-std=c++17", "--offload-arch=gfx950",
+                    "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "dooms_amd", "csrc"), src,
+                    "-o", str(exe)], check=True, capture_output=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+    assert "0 failures" in r.stdout
+
+
 def test_gemm_load_rows(tmp_path):
     # the rows the 128 x 128 GEMM's loads read (mx_kernels.hpp: gemm_load_row), by tests/cpp/gemm_rows_check.cpp
     exe = tmp_path / "gemm_rows_check"

@@ -201,6 +201,16 @@ def test_gemm_big_tiles_ragged(device):
         rows=[0, 1, 255, 256, 511, 700, 1023, 1024, 1279, 1280, 1299])
 
 
+@pytest.mark.parametrize("M,N,K,opts", [
+    (1300, 8300, 2080, dict(norm=True, bias=True, accumulate=True)),  # 256 x 256 tiles
+    (1900, 5700, 1056, dict(accumulate=True, y_pad=4)),               # 256 x 192 tiles
+    (1900, 5704, 1056, dict(bias=True, out_f16=True)),
+])
+def test_gemm_large_tiles_odd_k(device, M, N, K, opts):
+    """K an odd multiple of 32 on the 256-row tiles: the last step of 64 columns is half padding."""
+    run(device, 15, M, N, K, rows=[0, 1, 255, 256, 1023, 1024, M - 2, M - 1], **opts)
+
+
 def test_gemm_mid_tiles_ragged(device):
     """Enough 256 x 128 tiles (but too few 256 x 256 ones) for the 256 x 128 GEMM: ragged M and N, 3 steps of 32
     columns, f16 output with bias."""
