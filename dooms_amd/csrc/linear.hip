@@ -405,12 +405,11 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
     uint32_t off[Loads];
 #pragma unroll
     for (int i = 0; i < Loads; i++) {
-        const int row = 8 * (i * kBigWaves + wave) + lane / 8;
-        const int r = row < kBM ? gemm_load_row(m0, row, p.M) - m0 : gemm_load_row(n0, row - kBM, p.N) - n0;
-        off[i] = (uint32_t)r * (uint32_t)(row < kBM ? kp : p.K) * 2 + 16 * ((lane % 8) ^ ((row >> 1) & 7));
+        const int j = i * kBigWaves + wave, row = gemm_block_row<kBK>(j, lane), chunk = gemm_block_chunk<kBK>(j, lane);
+        off[i] = row < kBM ? gemm_load_offset<uint32_t>(m0, row, p.M, kp, chunk) : gemm_load_offset<uint32_t>(n0, row - kBM, p.N, p.K, chunk);
     }
-    // HALF: what this lane's weight loads of the last step go back (its chunk is the same for all of them)
-    const uint32_t back = HALF && ((lane % 8) ^ ((4 * wave + lane / 16) & 7)) >= 4 ? 64 : 0;
+    // HALF: what this lane's weight loads of the last step go back (kBigWaves is even: every block of a wave has its swizzle)
+    const uint32_t back = HALF ? gemm_half_back(gemm_block_chunk<kBK>(wave, lane)) : 0;
     // loads I0 .. I1 - 1 of a step
     auto issue = [&](int step, auto I0C, auto I1C) __attribute__((always_inline)) {
         const int64_t k0 = (int64_t)step * kBK * 2;  // bytes
@@ -526,12 +525,13 @@ __global__ __launch_bounds__(kBigThreads, 1) void gemm_w192_kernel(LinearParams 
 // tile lies whole in LDS with its 16-byte chunks permuted by the row (chunk ^ r % 16, or ^ r / 2 % 8 with 128-byte rows): the
 // 16-byte operand reads of 16 rows at one chunk hit 16 distinct 4-bank groups. The weights are MFMA operand A, so that
 // a lane holds 4 consecutive outputs of one row (16-byte stores).
-// HALF: K is an odd multiple of 32, as in gemm_big_tile; the last part's last step is half padding.
-template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF, bool HALF>
+// HALF: K is an odd multiple of 32, as in gemm_big_tile; the last part's last step is half padding. WIDE: the tile's rows span
+// 4 GiB or more, so the lanes' offsets take 64 bits.
+template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF, bool HALF, bool WIDE>
 __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     constexpr int WN = kWaves / WM;                        // waves along the weight rows
     constexpr int MI = BM / WM / 16, NJ = BN / WN / 16;    // 16 x 16 MFMA tiles per wave
-    constexpr int CH = BK / 8, RPB = 64 / CH;              // 16-byte chunks per row, rows per 1 KB load block
+    constexpr int RPB = 512 / BK;                          // rows per 1 KB load block
     constexpr int XB = BM / RPB, WB = BN / RPB;            // load blocks of a step
     constexpr int LPS = (XB + WB) / kWaves;                // loads per wave and step
     constexpr int KS = BK / 32;                            // MFMA steps per K step
@@ -552,19 +552,16 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     const int kp = HALF ? p.K + 32 : p.K;
     const int steps = kp / BK, s0 = (int)((int64_t)split * steps / S), nk = (int)((int64_t)(split + 1) * steps / S) - s0;
 
-    // load block j = i kWaves + wave of a step: RPB rows x BK columns; lane l fills position l % CH of row l / CH with
-    // chunk (l % CH) ^ swizzle(row)
-    auto swz = [](int row) { return BK == 128 ? row & 15 : (row >> 1) & 7; };
+    // load block i kWaves + wave of a step (see gemm_block_row)
     const char * const xg = reinterpret_cast<const char *>(p.xh + (int64_t)m0 * kp);
     const char * const wg = reinterpret_cast<const char *>(p.w[mi] + (int64_t)n0 * p.K);
-    uint32_t off[LPS];
+    using Offset = std::conditional_t<WIDE, uint64_t, uint32_t>;
+    Offset off[LPS];
 #pragma unroll
     for (int i = 0; i < LPS; i++) {
-        const int j = i * kWaves + wave;
-        const bool isx = j < XB;
-        const int row = (isx ? j : j - XB) * RPB + lane / CH;
-        const int r = isx ? gemm_load_row(m0, row, p.M) - m0 : gemm_load_row(n0, row, p.N) - n0;
-        off[i] = (uint32_t)r * (uint32_t)(isx ? kp : p.K) * 2 + 16 * ((lane % CH) ^ swz(row));
+        const int j = i * kWaves + wave, jb = j < XB ? j : j - XB;
+        const int row = gemm_block_row<BK>(jb, lane), chunk = gemm_block_chunk<BK>(jb, lane);
+        off[i] = j < XB ? gemm_load_offset<Offset>(m0, row, p.M, kp, chunk) : gemm_load_offset<Offset>(n0, row, p.N, p.K, chunk);
     }
     auto issue = [&](int step, int buf) __attribute__((always_inline)) {
         const int64_t k0 = (int64_t)(s0 + step) * BK * 2;
@@ -573,8 +570,8 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
         for (int i = 0; i < LPS; i++) {
             const int j = i * kWaves + wave;
             const char * src = (j < XB ? xg : wg) + k0;
-            uint32_t o = off[i];
-            if (half_step && j >= XB && ((lane % CH) ^ swz((j - XB) * RPB + lane / CH)) >= 4) o -= 64;
+            Offset o = off[i];
+            if (half_step && j >= XB) o -= gemm_half_back(gemm_block_chunk<BK>(j - XB, lane));
             __builtin_amdgcn_global_load_lds(src + o, (__attribute__((address_space(3))) void *)&sm[buf][512 * j], 16, 0, 0);
         }
     };
@@ -586,7 +583,7 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     const int wm = wave / WN, wn = wave % WN, l16 = lane % 16, grp = lane / 16;
     uint32_t rd[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ks++) rd[ks] = (uint32_t)l16 * BK * 2 + 16 * ((4 * ks + grp) ^ swz(l16));
+    for (int ks = 0; ks < KS; ks++) rd[ks] = (uint32_t)l16 * BK * 2 + 16 * ((4 * ks + grp) ^ gemm_swizzle<BK>(l16));
     const uint32_t lds0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) half_t *)sm[0];
 #pragma unroll
     for (int a = 0; a < NBUF - 1; a++)
@@ -750,8 +747,10 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     }
 }
 
-template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF, bool HALF>
-__global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(LinearParams p) { gemm_split_tile<OUT16, BM, BN, WM, BK, NBUF, HALF>(p); }
+template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF, bool HALF, bool WIDE>
+__global__ __launch_bounds__(kThreads, 1) void gemm_split_kernel(LinearParams p) {
+    gemm_split_tile<OUT16, BM, BN, WM, BK, NBUF, HALF, WIDE>(p);
+}
 
 // The kernels of kGemmCfgs, by shape: f32 and f16 outputs, and those of a K that is an odd multiple of 32, for the shapes
 // that take one.
@@ -762,13 +761,13 @@ struct GemmKernels {
     void (*half32)(LinearParams);
     void (*half16)(LinearParams);
 };
-template <int BM, int BN, int WM, int BK, int NBUF>
+template <int BM, int BN, int WM, int BK, int NBUF, bool WIDE = false>
 constexpr GemmKernels split_kernels() {
-    GemmKernels k{kThreads, gemm_split_kernel<false, BM, BN, WM, BK, NBUF, false>, gemm_split_kernel<true, BM, BN, WM, BK, NBUF, false>,
-                  nullptr, nullptr};
+    GemmKernels k{kThreads, gemm_split_kernel<false, BM, BN, WM, BK, NBUF, false, WIDE>,
+                  gemm_split_kernel<true, BM, BN, WM, BK, NBUF, false, WIDE>, nullptr, nullptr};
     if constexpr (BK == 64) {
-        k.half32 = gemm_split_kernel<false, BM, BN, WM, BK, NBUF, true>;
-        k.half16 = gemm_split_kernel<true, BM, BN, WM, BK, NBUF, true>;
+        k.half32 = gemm_split_kernel<false, BM, BN, WM, BK, NBUF, true, WIDE>;
+        k.half16 = gemm_split_kernel<true, BM, BN, WM, BK, NBUF, true, WIDE>;
     }
     return k;
 }
@@ -784,6 +783,7 @@ const GemmKernels & gemm_kernels(int cfg) {
          gemm_w192_kernel<true, true>},
         {kBigThreads, gemm_big_kernel<false, false>, gemm_big_kernel<true, false>, gemm_big_kernel<false, true>,
          gemm_big_kernel<true, true>},
+        split_kernels<64, 64, 2, 64, 4, true>(),
     };
     return kernels[cfg];
 }

@@ -23,6 +23,7 @@ namespace mx {
 struct GemmCfg {
     int bm, bn, bk, per_cu;
     float step1, step2, tile, merge, part_mb;
+    bool wide = false;  // 64-bit offsets within a tile
 };
 constexpr int kGemmCUs = 256;
 constexpr int kGemmBigRows = 256;  // rows of the tiles of 8 waves, which take whole K only
@@ -36,11 +37,19 @@ constexpr GemmCfg kGemmCfgs[] = {
     {128, 128, 64, 2, 0.887f, 1.078f, 0.f, 1.092f, 0.306f},
     {256, 192, 64, 1, 1.243f, 0.f, 5.946f, 0.f, 0.f},
     {256, 256, 64, 1, 1.426f, 0.f, 8.941f, 0.f, 0.f},
+    {64, 64, 64, 2, 0.340f, 0.553f, 0.f, 0.920f, 0.415f, true},
 };
 constexpr int kNumGemmCfgs = sizeof kGemmCfgs / sizeof *kGemmCfgs;
 
-// Whether shape c takes a K (a multiple of 32): the 64-column shapes take any, so that some shape always applies.
-inline bool gemm_takes(const GemmCfg & c, int32_t K) { return K % (c.bk == 128 ? 128 : 32) == 0; }
+// Whether the bytes from a tile's first row to any of its loads fit 32 bits.
+inline bool gemm_offsets_fit(const GemmCfg & c, int32_t K) {
+    return ((uint64_t)std::max(c.bm, c.bn) - 1) * (((uint64_t)K + 63) / 64 * 128) + 2 * c.bk <= UINT32_MAX;
+}
+// Whether shape c takes a K (a multiple of 32): the 64-column shapes take any that its offsets allow, and the wide one the
+// rest (K above 34 million), so that some shape always applies.
+inline bool gemm_takes(const GemmCfg & c, int32_t K) {
+    return K % (c.bk == 128 ? 128 : 32) == 0 && gemm_offsets_fit(c, K) != c.wide;
+}
 
 // counters of a split GEMM, each on a 256-byte line of its own
 inline size_t linear_counter_bytes(const LinearPlan & l) { return l.splits > 1 ? (size_t)l.tiles * kCounterStride * 4 : 0; }

@@ -200,6 +200,28 @@ __host__ __device__ inline int32_t gemm_load_row(int32_t first, int32_t row, int
     return first + row < rows - 1 ? first + row : rows - 1;
 }
 
+// A GEMM tile's operands are loaded in blocks of 1 KB: 512 / BK rows of BK columns. Lane l of block j fills 16-byte position
+// l % (BK / 8) of tile row (512 / BK) j + l / (BK / 8) in LDS with the row's chunk position ^ gemm_swizzle(row).
+template <int BK>
+__host__ __device__ inline int32_t gemm_swizzle(int32_t row) {
+    return BK == 128 ? row & 15 : (row >> 1) & 7;
+}
+template <int BK>
+__host__ __device__ inline int32_t gemm_block_row(int32_t block, int32_t lane) {
+    return block * (512 / BK) + lane / (BK / 8);
+}
+template <int BK>
+__host__ __device__ inline int32_t gemm_block_chunk(int32_t block, int32_t lane) {
+    return (lane % (BK / 8)) ^ gemm_swizzle<BK>(gemm_block_row<BK>(block, lane));
+}
+// Bytes from the operand's row `first` to that load in the first step (stride: halves between the operand's rows).
+template <typename O>
+__host__ __device__ inline O gemm_load_offset(int32_t first, int32_t row, int32_t rows, int32_t stride, int32_t chunk) {
+    return (O)(gemm_load_row(first, row, rows) - first) * (O)stride * 2 + 16 * (O)chunk;
+}
+// The last step of a K that is an odd multiple of 32: bytes that a weight load goes back, into the row's last chunks.
+__host__ __device__ inline uint32_t gemm_half_back(int32_t chunk) { return chunk >= 4 ? 64 : 0; }
+
 // How a product of more than kLinearGemvMaxRows rows runs.
 struct LinearPlan {
     int32_t cfg;     // the GEMM's tile shape

@@ -23,6 +23,14 @@ int main() {
                 const int a = linear_plan(M, N, K, 1, SIZE_MAX).cfg, b = linear_plan(M, N, K + 32, 1, SIZE_MAX).cfg;
                 CHECK(kGemmCfgs[b].bm != 256 || kGemmCfgs[a].bm == 256, "%d x %d x %d: shape %d, with K + 32 %d", M, N, K, a, b);
             }
+    // some shape takes every K, and none whose loads reach past 32 bits of a tile's first row without 64-bit offsets
+    for (int64_t K = 32; K <= INT32_MAX; K = K < 4096 ? K + 32 : K + K / 64 / 32 * 32 + 32) {
+        const int i = linear_plan(9, 64, (int32_t)K, 1, SIZE_MAX).cfg;
+        CHECK(i >= 0, "K %lld: no shape", (long long)K);
+        if (i >= 0 && !kGemmCfgs[i].wide)
+            CHECK((std::max(kGemmCfgs[i].bm, kGemmCfgs[i].bn) - 1) * (K + 63) / 64 * 128 + 2 * kGemmCfgs[i].bk <= UINT32_MAX, "K %lld: shape %d",
+                  (long long)K, i);
+    }
     std::printf("%d failures\n", failures);
     return failures != 0;
 }

@@ -425,10 +425,11 @@ def test_linear_plan(tmp_path):
 
 
 def test_gemm_load_rows(tmp_path):
-    # the rows the 128 x 128 GEMM's loads read (mx_kernels.hpp: gemm_load_row), by tests/cpp/gemm_rows_check.cpp
+    # the addresses of the GEMMs' operand loads (mx_kernels.hpp), by tests/cpp/gemm_rows_check.cpp
     exe = tmp_path / "gemm_rows_check"
     src = os.path.join(ROOT, "tests", "cpp", "gemm_rows_check.cpp")
-    subprocess.run(["/opt/rocm/bin/hipcc", "-O2", "-std=c++17", "--offload-arch=gfx950",
+    subprocess.run(["/opt/rocm/bin/hipcc", "-O2", "-std=c++17", "--offload-arch=gfx950", "-I", os.path.join(ROOT, "include"),
                     "-I", os.path.join(ROOT, "dooms_amd", "csrc"), src, "-o", str(exe)], check=True, capture_output=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
+    assert "0 failures" in r.stdout

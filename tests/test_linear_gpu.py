@@ -235,6 +235,25 @@ def test_gemm_tiles_ragged_k64_steps(device, M, N, opts, K):
     run(device, 13 + K, M, N, K, rows=[0, 1, 255, 256, 1023, 1024, M - 2, M - 1], **opts)
 
 
+@pytest.mark.parametrize("M,N,K", [(9, 132, 18_000_000), (40, 64, 36_000_032), (9, 64, 36_000_000)])
+def test_gemm_rows_far_apart(device, M, N, K):
+    """Rows so long that a tile's last ones lie 4 GiB or more behind its first. A handful of weights per row, each a power
+    of two in a column of its own, and whole inputs up to 16: every sum is exact."""
+    g = torch.Generator(device=device)
+    g.manual_seed(N)
+    x = torch.randint(1, 17, (M, K), generator=g, device=device, dtype=torch.int8).float()
+    w = torch.zeros(N, K, dtype=torch.float16, device=device)
+    cols = torch.randint(0, K, (N, 5), generator=g, device=device)
+    cols[:, 0] = K - 1 - torch.arange(N, device=device)  # the last step's columns too
+    cols[:, 1] = torch.arange(N, device=device)
+    ref = torch.zeros(M, N, dtype=torch.float64, device=device)
+    for i in range(5):
+        v = 2.0 ** (i - 2)
+        w[torch.arange(N, device=device), cols[:, i]] += v
+        ref += v * x[:, cols[:, i]].double()
+    assert torch.equal(A.linear(x, w).double(), ref)
+
+
 def test_gemm_llama3_attn_output_chunk(device):
     run(device, 7, 300, 4096, 4096, accumulate=True, rows=[0, 1, 127, 128, 255, 299])
 
