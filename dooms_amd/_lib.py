@@ -23,6 +23,7 @@ CODE_NAMES = {OK: "OK", INVALID_ARGUMENT: "INVALID_ARGUMENT", UNSUPPORTED: "UNSU
 EXPORTS = ("mx_attn_abi_version", "mx_attn_last_error", "mx_attn_prefill", "mx_attn_prefill_ws",
            "mx_attn_prefill_workspace_bytes", "mx_attn_prefill_rope", "mx_attn_prefill_rope_ws", "mx_attn_decode",
            "mx_attn_decode_f32", "mx_attn_decode_noalloc", "mx_attn_decode_rope", "mx_linear", "mx_linear_workspace_bytes",
+           "mx_linear_call_workspace_bytes",
            "mx_attn_decode_workspace_bytes", "mx_attn_decode_workspace_init", "mx_self_attention",
            "mx_self_attention_workspace_bytes")
 
@@ -119,6 +120,8 @@ def lib() -> ctypes.CDLL:
                                           P, P, ctypes.c_size_t, P]
         L.mx_linear_workspace_bytes.restype = ctypes.c_size_t
         L.mx_linear_workspace_bytes.argtypes = [ctypes.POINTER(MxLinearDesc)]
+        L.mx_linear_call_workspace_bytes.restype = ctypes.c_size_t
+        L.mx_linear_call_workspace_bytes.argtypes = [ctypes.POINTER(MxLinearDesc), ctypes.c_int32]
         L.mx_linear.restype = ctypes.c_int32
         L.mx_linear.argtypes = [ctypes.POINTER(MxLinearDesc), ctypes.c_int32, ctypes.POINTER(P), P, ctypes.POINTER(P),
                                 P, ctypes.POINTER(P), P, ctypes.c_size_t, P]
@@ -259,6 +262,10 @@ def linear_raw(desc: MxLinearDesc, w_ptrs, x: int, y_ptrs, gamma: int, bias_ptrs
 
 def linear_workspace_bytes(desc: MxLinearDesc) -> int:
     return lib().mx_linear_workspace_bytes(ctypes.byref(desc))
+
+
+def linear_call_workspace_bytes(desc: MxLinearDesc, count: int) -> int:
+    return lib().mx_linear_call_workspace_bytes(ctypes.byref(desc), count)
 
 
 def self_attention_workspace_bytes(desc: MxSelfAttnDesc) -> int:

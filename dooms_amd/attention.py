@@ -48,7 +48,7 @@ def _native():
         from . import _native as ext
         ext.bind(*[ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in (
             "mx_attn_prefill_ws", "mx_attn_decode", "mx_attn_decode_f32", "mx_attn_decode_rope", "mx_attn_prefill_rope_ws",
-            "mx_linear_workspace_bytes", "mx_linear", "mx_self_attention_workspace_bytes", "mx_self_attention")])
+            "mx_linear_call_workspace_bytes", "mx_linear", "mx_self_attention_workspace_bytes", "mx_self_attention")])
         _bound, _ext = L, ext
     return _ext
 
@@ -265,7 +265,7 @@ def linear(x, weights, *, out=None, gamma=None, bias=None, eps=1e-5, accumulate=
              (_lib.LINEAR_BIAS if bl is not None else 0) | (_lib.LINEAR_OUT_F16 if out_f16 else 0))
     d = _lib.MxLinearDesc(M=x.shape[0], N=N, K=K, flags=flags, x_stride=x.stride(0), y_stride=outs[0].stride(0),
                           eps=eps, reserved=0)
-    need = _lib.linear_workspace_bytes(d)
+    need = _lib.linear_call_workspace_bytes(d, len(ws_list))
     ws = torch.empty(max(need, 256), dtype=torch.uint8, device=x.device) if need else None
     _lib.check(_lib.linear_raw(d, [w.data_ptr() for w in ws_list], x.data_ptr(), [o.data_ptr() for o in outs],
                                gamma.data_ptr() if gamma is not None else 0,

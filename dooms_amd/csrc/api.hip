@@ -1102,7 +1102,13 @@ MX_ATTN_API size_t mx_linear_workspace_bytes(const mx_linear_desc * desc) {
     }
     const size_t rows = linear_ws_bytes(*desc);
     if (!rows || desc->N < 1 || desc->K < 1) return rows;
-    return rows + mx::linear_plan(desc->M, desc->N, desc->K, 1, SIZE_MAX).bytes;
+    return rows + mx::linear_plan_room(desc->M, desc->N, desc->K, 1);
+}
+
+MX_ATTN_API size_t mx_linear_call_workspace_bytes(const mx_linear_desc * desc, int32_t count) {
+    if (check_linear_desc(desc, count)) return 0;
+    const size_t rows = linear_ws_bytes(*desc);
+    return rows ? rows + mx::linear_plan(desc->M, desc->N, desc->K, count, SIZE_MAX).bytes : 0;
 }
 
 MX_ATTN_API int32_t mx_linear(const mx_linear_desc * desc, int32_t count, const uint16_t * const * W, const float * X,

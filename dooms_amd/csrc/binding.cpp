@@ -31,7 +31,7 @@ struct Api {
     decltype(&mx_attn_decode_f32) decode_f32 = nullptr;
     decltype(&mx_attn_decode_rope) decode_rope = nullptr;
     decltype(&mx_attn_prefill_rope_ws) prefill_rope_ws = nullptr;
-    decltype(&mx_linear_workspace_bytes) linear_workspace_bytes = nullptr;
+    decltype(&mx_linear_call_workspace_bytes) linear_workspace_bytes = nullptr;
     decltype(&mx_linear) linear = nullptr;
     decltype(&mx_self_attention_workspace_bytes) self_attention_workspace_bytes = nullptr;
     decltype(&mx_self_attention) self_attention = nullptr;
@@ -322,7 +322,7 @@ PyObject * linear(PyObject * const * a) {
     d.x_stride = x.stride(0);
     d.y_stride = outs[0].stride(0);
     d.eps = (float)real(a[5]);
-    const size_t bytes = api.linear_workspace_bytes(&d);
+    const size_t bytes = api.linear_workspace_bytes(&d, (int32_t)n);
     const at::Tensor work = bytes ? at::empty({(int64_t)std::max<size_t>(bytes, 256)}, x.options().dtype(at::kByte)) : at::Tensor();
     int32_t rc;
     {

@@ -93,4 +93,17 @@ inline LinearPlan linear_plan(int32_t M, int32_t N, int32_t K, int32_t count, si
     return best;
 }
 
+// The most that linear_plan takes behind the staged rows of a product of up to M rows. It does not grow with M (a product of
+// few rows has more parts), and depends on M through the tiles alone, so every 16th row count is looked at, up to the
+// last one at which some shape could be split.
+inline size_t linear_plan_room(int32_t M, int32_t N, int32_t K, int32_t count) {
+    int64_t top = 0;
+    for (const GemmCfg & c : kGemmCfgs)
+        if (c.merge > 0.f) top = std::max(top, c.bm * (kMaxSplitGrid / 2 / (count * (((int64_t)N + c.bn - 1) / c.bn))));
+    size_t room = 0;
+    for (int32_t m = (int32_t)std::min<int64_t>(M, top); m > kLinearGemvMaxRows; m = (m - 1) / 16 * 16)
+        room = std::max(room, linear_plan(m, N, K, count, SIZE_MAX).bytes);
+    return room;
+}
+
 }  // namespace mx

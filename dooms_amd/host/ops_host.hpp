@@ -103,16 +103,23 @@ private:
     DeviceBuffer ws_;
 };
 
-// One projection Y = X W^T of a decoder layer (flags MX_LINEAR_*), for up to max_rows input rows, on mx_linear's
-// kernels. Nothing allocates in run().
+// One projection Y = X W^T of a decoder layer (flags MX_LINEAR_*), for up to max_rows input rows and max_count matrices a
+// call, on mx_linear's kernels. Nothing allocates in run().
 class Projection {
 public:
     static Status create(int32_t N, int32_t K, uint32_t flags, float eps, int32_t max_rows, hipStream_t stream,
-                         std::unique_ptr<Projection> & out) {
-        if (N < 1 || K < 1 || max_rows < 1) return {Code::InvalidArgument, "N, K and max_rows must be >= 1"};
+                         std::unique_ptr<Projection> & out, int32_t max_count = 1) {
+        if (N < 1 || K < 1 || max_rows < 1 || max_count < 1)
+            return {Code::InvalidArgument, "N, K, max_rows and max_count must be >= 1"};
         std::unique_ptr<Projection> p(new Projection(N, K, flags, eps, stream));
         const mx_linear_desc d = p->desc(max_rows, K, N);
-        if (Status st = p->ws_.reserve(mx_linear_workspace_bytes(&d)); !st.is_ok()) return st;
+        size_t bytes = mx_linear_workspace_bytes(&d);
+        if (max_count > 1)  // (what a call takes behind its staged rows depends on the rows by sixteens)
+            for (int32_t m = max_rows; m > 8; m = (m - 1) / 16 * 16) {
+                const mx_linear_desc c = p->desc(m, K, (N + 7) / 8 * 8);
+                bytes = std::max(bytes, mx_linear_call_workspace_bytes(&c, max_count));
+            }
+        if (Status st = p->ws_.reserve(bytes); !st.is_ok()) return st;
         out = std::move(p);
         return {};
     }
@@ -157,7 +164,7 @@ public:
         if (c.n_layer < 1 || 2 * c.n_layer > 64) return {Code::InvalidArgument, "n_layer must be in [1, 32]"};
         std::unique_ptr<Projection> proj;
         if (Status st = Projection::create(c.n_state, c.n_state, MX_LINEAR_OUT_F16 | MX_LINEAR_BIAS, 0.f, c.n_audio_ctx,
-                                           stream, proj);
+                                           stream, proj, 2 * c.n_layer);
             !st.is_ok())
             return st;
         out.reset(new WhisperCrossCache(c, std::move(proj)));

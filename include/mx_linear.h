@@ -51,14 +51,22 @@ typedef struct mx_linear_desc {
 } mx_linear_desc;
 
 /*
- * Bytes of device workspace mx_linear asks for with this descriptor and one matrix; 0 for M <= 8. For M > 8:
- * M * round_up(K, 64) halves (256-byte rounded) for the input rows staged once as half(x * gamma * rms_scale) (the
- * values the reference's matmul stages per tile, with its rms_scale buffer folded in), and behind them, for products of
- * too few tiles to fill the chip, the partial tiles of a K cut into parts. The staged rows are what a call must have;
- * with less room behind them than asked for here it takes fewer parts (results agree within the summation order).
- * Nothing needs to be initialized, and nothing is kept between calls.
+ * Bytes of device workspace with which mx_linear runs any product of one matrix of up to desc->M rows at its best; 0 for
+ * M <= 8. For M > 8: M * round_up(K, 64) halves (256-byte rounded) for the input rows staged once as half(x * gamma *
+ * rms_scale) (the values the reference's matmul stages per tile, with its rms_scale buffer folded in), and behind them, for
+ * products of too few tiles to fill the chip, the partial tiles of a K cut into parts. The staged rows are what a call
+ * must have; with less room behind them than its plan asks for it takes fewer parts (results agree within the summation
+ * order). Nothing needs to be initialized, and nothing is kept between calls. Meant for sizing a workspace once: it
+ * looks at every row count up to M (tens of microseconds).
  */
 MX_ATTN_API size_t mx_linear_workspace_bytes(const mx_linear_desc * desc);
+
+/*
+ * Bytes of device workspace that one mx_linear call with exactly this descriptor and count matrices makes use of (staged
+ * rows and partial tiles as above); 0 for M <= 8, and for a descriptor or count that the call refuses. For callers that
+ * allocate per call.
+ */
+MX_ATTN_API size_t mx_linear_call_workspace_bytes(const mx_linear_desc * desc, int32_t count);
 
 /*
  * count products that share the input X and the shape: Y[i] = X W[i]^T (flags as desc). W, Y and bias are HOST arrays

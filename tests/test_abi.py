@@ -412,6 +412,31 @@ def test_decode_plan(tmp_path):
     assert r.returncode == 0, r.stdout
 
 
+@pytest.mark.parametrize("N,K", [(6144, 4096), (4096, 14336), (1152, 896), (1280, 1280), (64, 3584), (3584, 2080)])
+def test_linear_workspace_serves_fewer_rows(N, K):
+    """A workspace sized once holds what any call of fewer rows makes use of (those have more parts of K): the declared
+    size never shrinks with the rows, and is no smaller than the need of any call of up to that many."""
+    d = _lib.MxLinearDesc(M=0, N=N, K=K, flags=0, x_stride=K, y_stride=N, eps=0.0, reserved=0)
+    most = 0
+    for m in range(1, 1700):
+        d.M = m
+        need, sized = _lib.linear_call_workspace_bytes(d, 1), _lib.linear_workspace_bytes(d)
+        assert (need == 0) == (m <= 8) and (sized == 0) == (m <= 8)
+        most = max(most, need, sized)
+        assert sized == most, m
+
+
+def test_linear_call_workspace_of_several_matrices():
+    d = _lib.MxLinearDesc(M=16, N=4096, K=4096, flags=0, x_stride=4096, y_stride=4096, eps=0.0, reserved=0)
+    staged = 16 * 4096 * 2
+    one, two = _lib.linear_call_workspace_bytes(d, 1) - staged, _lib.linear_call_workspace_bytes(d, 2) - staged
+    assert one > 0 and two > 0  # both have K in parts
+    for count in (0, 65):
+        assert _lib.linear_call_workspace_bytes(d, count) == 0
+        assert "count" in _lib.last_error()
+    assert _lib.lib().mx_linear_call_workspace_bytes(None, 1) == 0
+
+
 def test_linear_plan(tmp_path):
     # the projections' plan (linear_plan.hpp), by tests/cpp/linear_plan_check.cpp
     exe = tmp_path / "linear_plan_check"
