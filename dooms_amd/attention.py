@@ -7,7 +7,9 @@ refused argument, here.
 """
 import contextlib
 import ctypes
+import importlib
 import math
+import warnings
 
 import torch
 
@@ -35,21 +37,42 @@ def _tuning(t):
     return _default_tuning if t is None else t
 
 
-_bound = None   # the library whose functions the extension holds
 _ext = None
+_bound = None   # the library whose functions the extension holds
+
+
+class _General:
+    """Stands in for an extension that is not built: every call goes the general path."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
 
 
 def _native():
     """dooms_amd._native (csrc/binding.cpp), the plain case of the entry points below in C++: each of its functions
-    returns what its namesake here does, a code of the library as an int, or None where the general path has to run."""
+    returns what its namesake here does, a code of the library as an int, or None where the general path has to run.
+    Without the extension every call goes that way, some 10 us slower; one built for other headers or another torch is
+    refused."""
     global _bound, _ext
     L = _lib.lib()
     if _bound is not L:
-        from . import _native as ext
-        ext.bind(*[ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in (
-            "mx_attn_prefill_ws", "mx_attn_decode", "mx_attn_decode_f32", "mx_attn_decode_rope", "mx_attn_prefill_rope_ws",
-            "mx_linear_call_workspace_bytes", "mx_linear", "mx_self_attention_workspace_bytes", "mx_self_attention")])
-        _bound, _ext = L, ext
+        try:
+            ext = importlib.import_module("._native", __package__)
+        except ModuleNotFoundError:
+            warnings.warn("dooms_amd._native is not built (`python -m dooms_amd.build` does): calls take the slower general path",
+                          RuntimeWarning, stacklevel=3)
+            ext = _General()
+        except ImportError as e:
+            raise ImportError(f"{e}: build the extension for this torch with `python -m dooms_amd.build`") from e
+        else:
+            ext.bind(L.mx_attn_abi_version(),
+                     tuple(ctypes.sizeof(t) for t in (_lib.MxAttnDesc, _lib.MxAttnRope, _lib.MxLinearDesc, _lib.MxSelfAttnDesc)),
+                     *[ctypes.cast(getattr(L, f), ctypes.c_void_p).value for f in (
+                         "mx_attn_prefill_ws", "mx_attn_decode", "mx_attn_decode_f32", "mx_attn_decode_rope",
+                         "mx_attn_prefill_rope_ws", "mx_linear_call_workspace_bytes", "mx_linear",
+                         "mx_self_attention_workspace_bytes", "mx_self_attention")])
+        _ext = ext   # before _bound: another thread that finds the library bound finds the extension too
+        _bound = L
     return _ext
 
 

@@ -1,7 +1,9 @@
-"""Builds the gfx950 attention library libmx_attn.so in-tree with hipcc (no CUDA, no torch in the ABI)."""
+"""Builds the gfx950 attention library libmx_attn.so in-tree with hipcc (no CUDA, no torch in the ABI), and the torch front
+end's extension with it."""
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -27,8 +29,9 @@ def _run(cmd):
 
 
 def build(verbose: bool = False, out: str = LIB, defines=()) -> str:
-    """Compiles every HIP source (one hipcc per source, in parallel) and links dooms_amd/libmx_attn.so; returns its
-    path. Raises on a compile error. `out` and `defines` (extra -D macros) serve experiments that build variants."""
+    """Compiles every HIP source (one hipcc per source, in parallel) and links dooms_amd/libmx_attn.so, then builds the
+    extension against the same headers; returns the library's path. Raises on a compile error. `out` and `defines` (extra
+    -D macros) serve experiments that build variants of the library alone."""
     from concurrent.futures import ThreadPoolExecutor
     objdir = os.path.join(os.path.dirname(out), "_build", os.path.splitext(os.path.basename(out))[0])
     os.makedirs(objdir, exist_ok=True)
@@ -47,16 +50,17 @@ def build(verbose: bool = False, out: str = LIB, defines=()) -> str:
     if verbose and (msgs + msg).strip():
         print(msgs + msg, file=sys.stderr)
     os.replace(out + ".tmp", out)
+    if out == LIB:
+        build_binding()
     return out
 
 
-EXT = os.path.join(PKG, "_native.so")
+# the interpreter's own suffix: another Python does not see it and takes the general path
+EXT = os.path.join(PKG, "_native" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
 def build_binding(out: str = EXT) -> str:
     """The torch front end's extension (csrc/binding.cpp): host code only, against the headers of the torch in use."""
-    import sysconfig
-
     import torch
     root = os.path.dirname(torch.__file__)
     inc = [os.path.join(ROOT, "include"), os.path.join(root, "include"), "/opt/rocm/include", sysconfig.get_paths()["include"]]
@@ -99,7 +103,7 @@ def build_host_test() -> str:
 
 if __name__ == "__main__":
     print(build(verbose=True))
-    print(build_binding())
+    print(EXT)
 
 
 SAN_DIR = os.path.join(ROOT, "tests", "cpp", "_san")

@@ -383,10 +383,24 @@ PyObject * entry(PyObject *, PyObject * const * args, Py_ssize_t n) {
     }
 }
 
-// bind(addresses): the library's functions in the order of Api
+// bind(abi version, (sizes of mx_attn_desc, mx_attn_rope, mx_linear_desc, mx_self_attn_desc), addresses): the library's
+// functions in the order of Api. A library of another version, or descriptors of another layout than this extension was
+// compiled with, are refused.
 PyObject * bind(PyObject *, PyObject * args) {
+    int version;
+    Py_ssize_t size[4];
     unsigned long long p[9];
-    if (!PyArg_ParseTuple(args, "KKKKKKKKK", p, p + 1, p + 2, p + 3, p + 4, p + 5, p + 6, p + 7, p + 8)) return nullptr;
+    if (!PyArg_ParseTuple(args, "i(nnnn)KKKKKKKKK", &version, size, size + 1, size + 2, size + 3, p, p + 1, p + 2, p + 3, p + 4, p + 5, p + 6, p + 7,
+                          p + 8))
+        return nullptr;
+    const size_t own[4] = {sizeof(mx_attn_desc), sizeof(mx_attn_rope), sizeof(mx_linear_desc), sizeof(mx_self_attn_desc)};
+    bool same = version == MX_ATTN_ABI_VERSION;
+    for (int i = 0; i < 4; i++) same = same && (size_t)size[i] == own[i];
+    if (!same) {
+        PyErr_Format(PyExc_ImportError, "dooms_amd._native was built for version %d of the library, which is %d, or for other descriptors: build "
+                     "both with `python -m dooms_amd.build`", (int)MX_ATTN_ABI_VERSION, version);
+        return nullptr;
+    }
     auto set = [](auto & f, unsigned long long v) { f = reinterpret_cast<std::remove_reference_t<decltype(f)>>((uintptr_t)v); };
     set(api.prefill_ws, p[0]);
     set(api.decode, p[1]);
