@@ -78,8 +78,9 @@ LIB_TRACE = os.path.join(os.path.dirname(LIB), "libmx_attn_trace.so")
 
 
 def build_trace(verbose: bool = False) -> str:
-    """The phase-trace variant of the library (MX_ATTN_TRACE: the decode kernel stamps its phases per workgroup and
-    exports mx_attn_trace_read), used by `bench.py --trace-decode`; the product library compiles the stamps away."""
+    """The diagnostic variant of the library (MX_ATTN_TRACE): the decode kernel stamps its phases per workgroup and exports
+    mx_attn_trace_read, used by `bench.py --trace-decode` (the product library compiles the stamps away), and projections can
+    be run on a given tile shape (mx_linear_trace_run), used by the tests of those kernels."""
     return build(verbose=verbose, out=LIB_TRACE, defines=("MX_ATTN_TRACE=1",))
 
 

@@ -784,10 +784,11 @@ int32_t check_linear_desc(const mx_linear_desc * desc, int32_t count) {
     return MX_ATTN_OK;
 }
 
-// Checks of an mx_linear call and its kernel parameters (for M == 0 only the descriptor is checked).
+// Checks of an mx_linear call and its kernel parameters (for M == 0 only the descriptor is checked). forced: a plan to run
+// instead of linear_plan's.
 int32_t linear_params(const mx_linear_desc * desc, int32_t count, const uint16_t * const * W, const float * X,
                       void * const * Y, const float * gamma, const float * const * bias, void * workspace,
-                      size_t ws_bytes, mx::LinearParams & p) {
+                      size_t ws_bytes, mx::LinearParams & p, const mx::LinearPlan * forced = nullptr) {
     if (int32_t rc = check_linear_desc(desc, count)) return rc;
     const mx_linear_desc & d = *desc;
     if (d.M == 0) return MX_ATTN_OK;
@@ -810,7 +811,9 @@ int32_t linear_params(const mx_linear_desc * desc, int32_t count, const uint16_t
     p.gamma = gamma;
     p.xh = static_cast<mx::half_t *>(workspace);
     p.plan = mx::LinearPlan{-1, 1, 0, 0};
-    if (need) p.plan = mx::linear_plan(d.M, d.N, d.K, count, ws_bytes - need);
+    if (need) p.plan = forced ? *forced : mx::linear_plan(d.M, d.N, d.K, count, ws_bytes - need);
+    if (p.plan.bytes > ws_bytes - need)
+        return fail(MX_ATTN_RESOURCE_EXHAUSTED, "workspace of %zu bytes is smaller than the %zu bytes needed", ws_bytes, need + p.plan.bytes);
     p.counters = reinterpret_cast<uint32_t *>(static_cast<char *>(workspace) + need);
     p.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + need + mx::linear_counter_bytes(p.plan));
     p.x_stride = d.x_stride;
@@ -1119,5 +1122,46 @@ MX_ATTN_API int32_t mx_linear(const mx_linear_desc * desc, int32_t count, const 
     if (desc->M == 0) return MX_ATTN_OK;
     return hip_status(mx::launch_linear(p, static_cast<hipStream_t>(stream)), "linear launch");
 }
+
+#ifdef MX_ATTN_TRACE
+// The diagnostic variant of the library also tells how a projection would run, and runs one on a tile shape and a number of
+// parts of the caller's choice, so that tests reach every shape whatever the costs say.
+
+// shape[0 .. 4]: rows, columns and K step of tile shape i, most parts of this K (0: the shape does not take it), whether its
+// offsets have 64 bits; returns the number of shapes.
+__attribute__((visibility("default"))) int32_t mx_linear_trace_shape(int32_t i, int32_t K, int32_t * shape) {
+    if (i >= 0 && i < mx::kNumGemmCfgs) {
+        const mx::GemmCfg & c = mx::kGemmCfgs[i];
+        const bool takes = K % (c.bk == 128 ? 128 : 32) == 0 && (c.wide || mx::gemm_offsets_fit(c, K));
+        shape[0] = c.bm;
+        shape[1] = c.bn;
+        shape[2] = c.bk;
+        shape[3] = !takes ? 0 : c.merge > 0.f ? std::min(mx::kMaxParts, (K + c.bk - 1) / c.bk) : 1;
+        shape[4] = c.wide;
+    }
+    return mx::kNumGemmCfgs;
+}
+
+// plan[0 .. 1]: the tile shape and the parts that mx_linear takes for this call with all the workspace that it asks for.
+__attribute__((visibility("default"))) void mx_linear_trace_plan(const mx_linear_desc * d, int32_t count, int32_t * plan) {
+    const mx::LinearPlan l = mx::linear_plan(d->M, d->N, d->K, count, SIZE_MAX);
+    plan[0] = l.cfg;
+    plan[1] = l.splits;
+}
+
+// mx_linear on tile shape i with K in the given number of parts.
+__attribute__((visibility("default"))) int32_t mx_linear_trace_run(
+    const mx_linear_desc * desc, int32_t count, const uint16_t * const * W, const float * X, void * const * Y, const float * gamma,
+    const float * const * bias, void * workspace, size_t ws_bytes, mx_attn_stream stream, int32_t i, int32_t parts) {
+    if (int32_t rc = check_linear_desc(desc, count)) return rc;
+    int32_t shape[5] = {};
+    if (desc->M <= mx::kLinearGemvMaxRows || i < 0 || i >= mx_linear_trace_shape(i, desc->K, shape) || parts < 1 || parts > shape[3])
+        return fail(MX_ATTN_INVALID_ARGUMENT, "tile shape %d does not take M %d, K %d in %d parts", i, desc->M, desc->K, parts);
+    const mx::LinearPlan plan = mx::linear_plan_of(i, parts, desc->M, desc->N, count);
+    mx::LinearParams p;
+    if (int32_t rc = linear_params(desc, count, W, X, Y, gamma, bias, workspace, ws_bytes, p, &plan)) return rc;
+    return hip_status(mx::launch_linear(p, static_cast<hipStream_t>(stream)), "linear launch");
+}
+#endif
 
 }  // extern "C"

@@ -374,3 +374,33 @@ def test_plan_loses_no_precision(device, H, G, hd, lens):
         err.append(float((out.double() - ref).norm() / ref.norm()))
     print(f"{H}/{G} {hd} {len(lens)} x {max(lens)}: {err[0]:.4e} against {err[1]:.4e}")
     assert err[0] <= 1.002 * err[1]
+
+
+@pytest.mark.parametrize("H,G,hd,n_q", [(28, 4, 128, 5), (14, 2, 64, 3), (20, 20, 64, 33), (32, 8, 128, 5), (9, 3, 64, 11), (6, 3, 256, 9)])
+@pytest.mark.parametrize("lens", [[300, 1100, 40], [129, 2500, 900, 60, 1700], [640 + 61 * i for i in range(12)], [5000, 4700, 4200, 4100]])
+@pytest.mark.parametrize("causal", [False, True])
+def test_ragged_batch_of_several_row_tiles(device, H, G, hd, n_q, lens, causal):
+    """More packed rows per kv head than a tile holds, over a ragged batch: each (split, kv head) group's row tiles on one
+    XCD, each sequence's groups starting on the XCD after the previous sequence's, f16 and f32 rows against f64."""
+    assert n_q * H // G > 16
+    g = torch.Generator(device=device)
+    g.manual_seed(sum(lens) + hd + n_q)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=device)
+    q = rnd(len(lens) * n_q, H * hd)
+    ks, vs = [rnd(n, G * hd).half() for n in lens], [rnd(n, G * hd).half() for n in lens]
+    refs, lses = [], []
+    for b, n in enumerate(lens):
+        qq = q[b * n_q:(b + 1) * n_q].half().double().view(n_q, G, H // G, hd)
+        kk, vv = ks[b].double().view(n, G, hd), vs[b].double().view(n, G, hd)
+        s = torch.stack([(qq[:, i].reshape(-1, hd) @ kk[:, i].T).view(n_q, H // G, n) for i in range(G)], 1) / hd ** 0.5
+        if causal:
+            past = torch.arange(n, device=device)[None] > n - n_q + torch.arange(n_q, device=device)[:, None]
+            s.masked_fill_(past[:, None, None], -float("inf"))
+        pr = torch.softmax(s, 3)
+        o = torch.stack([(pr[:, i].reshape(-1, n) @ vv[:, i]).view(n_q, H // G, hd) for i in range(G)], 1)
+        refs.append(o.reshape(n_q, H * hd))
+        lses.append(torch.logsumexp(s, 3).reshape(n_q, H))
+    ref, rl = torch.cat(refs).cpu().numpy(), torch.cat(lses).cpu().numpy()
+    for dt in (torch.float16, torch.float32):
+        out, lse = A.decode(q.to(dt), ks, vs, lens, n_head=H, n_head_kv=G, head_dim=hd, n_q=n_q, causal=causal, want_lse=True)
+        assert_close(out.float().cpu().numpy(), ref, hd, f"{lens} {dt}", lse.cpu().numpy(), rl)
