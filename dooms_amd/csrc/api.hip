@@ -204,6 +204,22 @@ DecodePlan decode_plan(const mx_attn_desc & d, const int32_t * kv_len, int n_seq
     return base;
 }
 
+// The order of a launch's sequences in its grid: the longest first, so that the workgroups past a shorter one's splits come
+// late (f16 rows in random order, us: 16 Llama-3-8B caches of 87-700 keys 13.3 -> 11.7, 16 Qwen2.5-7B caches of 1.3k-7.3k
+// 35.5 -> 33.1). Not on the XCD-mapped grid with more live workgroups than run at once (two per CU): later ones fill the
+// gaps there, and the sorted order ran up to 3 % slower (16 Llama-3-8B caches of 325-2600 keys 26.7 against 27.5). Equal
+// lengths keep the caller's order. By insertion: std::stable_sort takes a buffer from the heap, and a decode call must not.
+void decode_order(const int32_t * kv_len, int n_seq, int64_t wgs_per_split, int64_t chunk, bool xcd, int * order) {
+    int64_t live = 0;
+    for (int i = 0; i < n_seq; i++) live += (kv_len[i] + chunk - 1) / chunk * wgs_per_split;
+    const bool sort = !xcd || live <= 512;
+    for (int i = 0; i < n_seq; i++) {
+        int at = i;
+        for (; sort && at > 0 && kv_len[order[at - 1]] < kv_len[i]; at--) order[at] = order[at - 1];
+        order[at] = i;
+    }
+}
+
 // Workspace layout: kMaxTilesPerLaunch split counters (one per (sequence of a launch, kv head, row tile), each on a
 // 256-byte line of its own) at a fixed place, then the partials. The counters must be zero when a call starts, and
 // every call leaves the ones it used at zero; the partials are left as they are. So the counter region has the same
@@ -605,19 +621,12 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
         const DecodePlan plan = decode_plan(d, kv_len + b0, n_seq, s, f32);
         const int64_t chunk = plan.chunk;
         p.chunk = (int32_t)std::min<int64_t>(chunk, INT32_MAX / 2);
-        // The longest sequences first, so that the workgroups past a shorter one's splits come late (f16 rows in random
-        // order, us: 16 Llama-3-8B caches of 87-700 keys 13.3 -> 11.7, 16 Qwen2.5-7B caches of 1.3k-7.3k 35.5 -> 33.1). Not
-        // on the XCD-mapped grid with more live workgroups than run at once (two per CU): later ones fill the gaps
-        // there, and the sorted order ran up to 3 % slower (16 Llama-3-8B caches of 325-2600 keys 26.7 against 27.5).
-        int64_t live = 0;
-        for (int i = 0; i < n_seq; i++) live += (kv_len[b0 + i] + chunk - 1) / chunk * d.n_head_kv * s.n_rowtiles;
         int order[mx::kMaxSeqPerLaunch];
-        for (int i = 0; i < n_seq; i++) order[i] = b0 + i;
-        if (!p.xcd_heads || live <= 512) std::stable_sort(order, order + n_seq, [&](int x, int y) { return kv_len[x] > kv_len[y]; });
+        decode_order(kv_len + b0, n_seq, d.n_head_kv * s.n_rowtiles, chunk, p.xcd_heads, order);
         p.max_split = 1;
         int32_t groups = 0;
         for (int i = 0; i < n_seq; i++) {
-            const int32_t b = order[i], n = kv_len[b];
+            const int32_t b = b0 + order[i], n = kv_len[b];
             p.seq[i].k = static_cast<const mx::half_t *>(k_caches[b]);
             p.seq[i].v = static_cast<const mx::half_t *>(v_caches[b]);
             p.seq[i].len = n;

@@ -1,9 +1,45 @@
-// CPU check of the decode split plan (api.hip: decode_plan), over batches of sequences of up to 256 keys.
+// CPU check of the decode split plan (api.hip: decode_plan), over batches of sequences of up to 256 keys, and of the order
+// of a launch's sequences (decode_order).
 #include "../../dooms_amd/csrc/api.hip"
 
+#include <cstdlib>
+#include <numeric>
+#include <random>
 #include <vector>
 
+static int allocations = 0;
+void * operator new(size_t n) {
+    allocations++;
+    return std::malloc(n);
+}
+void * operator new(size_t n, const std::nothrow_t &) noexcept { return operator new(n); }
+void operator delete(void * p) noexcept { std::free(p); }
+void operator delete(void * p, size_t) noexcept { std::free(p); }
+
+// The longest first, equal lengths as they come, and nothing taken from the heap; on the XCD-mapped grid only with at most
+// 512 live workgroups.
+static bool order_ok(const std::vector<int32_t> & lens, bool xcd, int64_t chunk) {
+    int64_t live = 0;
+    for (int32_t n : lens) live += 8 * ((n + chunk - 1) / chunk);
+    std::vector<int> want(lens.size());
+    std::iota(want.begin(), want.end(), 0);
+    if (!xcd || live <= 512) std::stable_sort(want.begin(), want.end(), [&](int a, int b) { return lens[a] > lens[b]; });
+    int got[mx::kMaxSeqPerLaunch];
+    const int before = allocations;
+    decode_order(lens.data(), (int)lens.size(), 8, chunk, xcd, got);
+    return allocations == before && std::equal(want.begin(), want.end(), got);
+}
+
 int main() {
+    std::mt19937 rng(1);
+    for (int t = 0; t < 4000; t++) {
+        std::vector<int32_t> lens(1 + rng() % mx::kMaxSeqPerLaunch);
+        for (int32_t & n : lens) n = 1 + rng() % (t % 2 ? 9000 : 5);
+        if (!order_ok(lens, t % 4 >= 2, 128)) {
+            std::printf("the order of %zu sequences\n", lens.size());
+            return 1;
+        }
+    }
     // Whole sequences run on workgroups of 8 waves, of which a CU holds one on f32 rows (two waves per SIMD): at head dim 64
     // they are taken only where every workgroup has a CU of its own, else a second round costs more than the merge. Where
     // splits of 128 keys pass the workgroup cap, the sequences are whole on 4 waves.
