@@ -644,6 +644,14 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
         // 2048 keys, two XCDs streaming) measured 5.87 -> 6.02, Whisper cross-attention (12 splits, 7.7 MB) no gain.
         if (n_seq == 1 && p.max_split <= 8 && kv_bytes <= ((int64_t)4 << 20)) p.xcd_heads = 1;
         if (p.max_split > 32) p.xcd_heads = 0;  // the XCD-local counter counts at most 63 splits per XCD field
+        // One row tile and the same splits for every sequence, not on the XCD-mapped grid: each sequence's row of the grid
+        // holds its workgroups only, which then spread over the XCDs by themselves. Padded to whole XCD rounds, the
+        // workgroups that end at once upset the dealing of the others, and near a full round one CU too many got two
+        // (12 sequences of 132-256 keys of 20 kv heads, whole, us: f16 of head dim 128 12.4 -> 8.6, 10.3 split in two;
+        // the fused step at head dim 64 10.2 -> 7.2, 8.5 split; of 900 batches up to 512 workgroups a fifth were slower whole
+        // than split, none is now).
+        p.exact = !p.xcd_heads && s.n_rowtiles == 1 && groups == p.max_split * d.n_head_kv * n_seq;
+        for (int i = 0; p.exact && i < n_seq; i++) p.seq[i].xcd0 = 0;
         if (int32_t rc = hip_status(mx::launch_decode(p, n_seq, d.head_dim, s.rt, plan.waves, st), "decode launch")) return rc;
     }
     return MX_ATTN_OK;

@@ -404,3 +404,18 @@ def test_ragged_batch_of_several_row_tiles(device, H, G, hd, n_q, lens, causal):
     for dt in (torch.float16, torch.float32):
         out, lse = A.decode(q.to(dt), ks, vs, lens, n_head=H, n_head_kv=G, head_dim=hd, n_q=n_q, causal=causal, want_lse=True)
         assert_close(out.float().cpu().numpy(), ref, hd, f"{lens} {dt}", lse.cpu().numpy(), rl)
+
+
+# sequences of the same number of splits, kv heads that are no multiple of 8: the grid holds their workgroups only
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("H,G,hd", [(1, 1, 64), (9, 3, 128), (20, 20, 64), (35, 5, 128), (28, 7, 64), (9, 9, 256)])
+@pytest.mark.parametrize("lens", [[130, 256, 180], [40, 128], [300, 257, 384, 290, 301], [1400, 1281, 1350], [256 - 3 * i for i in range(32)]])
+def test_equal_splits(device, H, G, hd, lens, f32):
+    rng = np.random.default_rng(lens[0] + G)
+    q = torch.from_numpy(normal_f16(rng, (len(lens), H * hd), 1.0))
+    caches = [[normal_f16(rng, (n, G * hd), 1.0) for _ in range(2)] for n in lens]
+    ks, vs = ([torch.from_numpy(c[i]).to(device) for c in caches] for i in range(2))
+    out, lse = A.decode(q.to(device, torch.float32 if f32 else torch.float16), ks, vs, lens, n_head=H, n_head_kv=G, head_dim=hd, want_lse=True)
+    for b, n in enumerate(lens):
+        ro, rl = ref_attention(q[b:b + 1].numpy(), *caches[b], H, G, hd, 1.0 / np.sqrt(hd), p0=n - 1, causal=False)
+        assert_close(out[b:b + 1].cpu().numpy().astype(np.float64), ro, hd, f"sequence {b} of {n} keys", lse[b:b + 1].cpu().numpy(), rl)
