@@ -144,7 +144,9 @@ DecodeShape decode_shape(const mx_attn_desc * d) {
 //     8.1 whole; f16 rows fit two and stay ahead: 16 x 140 keys 7.6 -> 6.4), nor where the workgroup cap leaves the
 //     sequences whole anyway, on 4 waves (32 x 140 keys of 28 kv heads, f16, 10.6 on 4 waves, 12.1 on 8);
 //   * head dim 64, several sequences: at most 16 splits, the most that one round of the merge folds, with twice the
-//     waves per split (3 x 3096 keys of 2 kv heads 10.8 -> 10.1).
+//     waves per split (3 x 3096 keys of 2 kv heads 10.8 -> 10.1). On f32 rows a CU holds one such workgroup: where the
+//     sequences differ in their splits, whose shares of the grid are then padded, only up to 128 of them (500 ragged
+//     batches: above 160 workgroups up to 1.26x slower than with 128-key splits, up to 160 1.02x).
 struct DecodePlan {
     int64_t chunk;
     int waves;
@@ -199,7 +201,9 @@ DecodePlan decode_plan(const mx_attn_desc & d, const int32_t * kv_len, int n_seq
         return {2 * quantum, 8};
     if (d.head_dim == 64 && n_seq > 1 && lmax <= 16 * 640) {
         const DecodePlan few = plan(16);
-        if (few.chunk * base.waves <= base.chunk * few.waves) return few;  // no more keys per wave
+        const bool equal = (lmin + few.chunk - 1) / few.chunk == (lmax + few.chunk - 1) / few.chunk;
+        if (few.chunk * base.waves <= base.chunk * few.waves && (!f32 || equal || launch_wgs(few.chunk) <= 128))
+            return few;  // no more keys per wave
     }
     return base;
 }

@@ -61,5 +61,23 @@ int main() {
                         return 1;
                     }
                 }
+    // f32 rows of head dim 64 take 16 splits of 8 waves up to one workgroup per CU, in a ragged batch up to half of that
+    for (int n_seq = 2; n_seq <= mx::kMaxSeqPerLaunch; n_seq++)
+        for (int heads : {1, 2, 3, 4, 8, 20})
+            for (int last : {4000, 1700}) {
+                mx_attn_desc d{};
+                d.n_head = d.n_head_kv = heads;
+                d.head_dim = 64;
+                d.n_q = 1;
+                std::vector<int32_t> lens(n_seq, 4000);
+                lens.back() = last;
+                const DecodePlan plan = decode_plan(d, lens.data(), n_seq, DecodeShape{1, 4, 1}, true);
+                const int wgs = heads * ((n_seq - 1) * 16 + (last + 255) / 256);
+                if (wgs <= 512 && plan.waves != (wgs <= (last == 4000 ? 256 : 128) ? 8 : 4)) {
+                    std::printf("%d sequences of 4000 and %d keys, %d heads: %lld keys per split, %d waves\n", n_seq, last, heads,
+                                (long long)plan.chunk, plan.waves);
+                    return 1;
+                }
+            }
     return 0;
 }
