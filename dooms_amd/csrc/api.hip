@@ -208,15 +208,24 @@ DecodePlan decode_plan(const mx_attn_desc & d, const int32_t * kv_len, int n_seq
     return base;
 }
 
+// The 4-wave head-dim-128 kernels on f32 rows run one workgroup per CU in launches well below one per CU. Two fit a CU (the
+// bound on their registers, decode.hip), but the padding of the sequences' shares of a ragged batch's grid then deals two
+// to some CUs and none to others: of 200 such launches those of 128 workgroups and more were up to 1.19x slower than one
+// by one, 2 % on average (4 sequences of 471 to 1773 keys of Llama-3-8B, fused step, 9.0 us against 10.1). Nearer to one per
+// CU two are ahead, as one CU too many has to take a second one after the first: 13 to 23 % from 192 off the XCD-mapped
+// grid, 3 to 13 % from 224 on it (single launches up to 14 % behind).
+bool decode_alone(bool f32, int head_dim, int waves, int64_t live, bool xcd) {
+    return f32 && head_dim == 128 && waves == 4 && live < (xcd ? 224 : 192);
+}
+
 // The order of a launch's sequences in its grid: the longest first, so that the workgroups past a shorter one's splits come
 // late (f16 rows in random order, us: 16 Llama-3-8B caches of 87-700 keys 13.3 -> 11.7, 16 Qwen2.5-7B caches of 1.3k-7.3k
-// 35.5 -> 33.1). Not on the XCD-mapped grid with more live workgroups than run at once (two per CU): later ones fill the
-// gaps there, and the sorted order ran up to 3 % slower (16 Llama-3-8B caches of 325-2600 keys 26.7 against 27.5). Equal
-// lengths keep the caller's order. By insertion: std::stable_sort takes a buffer from the heap, and a decode call must not.
-void decode_order(const int32_t * kv_len, int n_seq, int64_t wgs_per_split, int64_t chunk, bool xcd, int * order) {
-    int64_t live = 0;
-    for (int i = 0; i < n_seq; i++) live += (kv_len[i] + chunk - 1) / chunk * wgs_per_split;
-    const bool sort = !xcd || live <= 512;
+// 35.5 -> 33.1). On the XCD-mapped grid not with more live workgroups than run at once (two per CU: later ones fill the
+// gaps there, and the sorted order ran up to 3 % slower, 16 Llama-3-8B caches of 325-2600 keys 26.7 against 27.5), nor with
+// one per CU (decode_alone: level on average, at worst 1.04x). Equal lengths keep the caller's order. By insertion:
+// std::stable_sort takes a buffer from the heap, and a decode call must not.
+void decode_order(const int32_t * kv_len, int n_seq, int64_t live, bool xcd, bool alone, int * order) {
+    const bool sort = !xcd || (live <= 512 && !alone);
     for (int i = 0; i < n_seq; i++) {
         int at = i;
         for (; sort && at > 0 && kv_len[order[at - 1]] < kv_len[i]; at--) order[at] = order[at - 1];
@@ -625,8 +634,11 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
         const DecodePlan plan = decode_plan(d, kv_len + b0, n_seq, s, f32);
         const int64_t chunk = plan.chunk;
         p.chunk = (int32_t)std::min<int64_t>(chunk, INT32_MAX / 2);
+        int64_t live = 0;
+        for (int i = 0; i < n_seq; i++) live += (kv_len[b0 + i] + chunk - 1) / chunk * d.n_head_kv * s.n_rowtiles;
+        p.alone = decode_alone(f32, d.head_dim, plan.waves, live, p.xcd_heads);
         int order[mx::kMaxSeqPerLaunch];
-        decode_order(kv_len + b0, n_seq, d.n_head_kv * s.n_rowtiles, chunk, p.xcd_heads, order);
+        decode_order(kv_len + b0, n_seq, live, p.xcd_heads, p.alone, order);
         p.max_split = 1;
         int32_t groups = 0;
         for (int i = 0; i < n_seq; i++) {

@@ -236,7 +236,7 @@ __device__ __forceinline__ void merge_wide(const DecodeParams & p, const float *
 // are used from registers for that position and written into the caches by the one workgroup whose split holds it.
 // NT: the keys and values are loaded non-temporally (p.kv_nt: a launch whose K/V stream from HBM once).
 // Head dim 128: two waves per SIMD at least. Without the bound the f32 variants of 4 waves took 288 registers, one wave
-// per SIMD, and a launch of more workgroups than CUs ran them in twice the rounds.
+// per SIMD, and a launch of more workgroups than CUs ran them in twice the rounds (fewer run one per CU all the same: p.alone).
 template <int HD, int RT, bool F32, int NW, bool NT = false>
 __global__ __launch_bounds__(NW * kWave) __attribute__((amdgpu_waves_per_eu(HD == 128 || NW == 8 ? 2 : 1)))
 void decode_kernel(DecodeParams p) {
@@ -769,26 +769,29 @@ void decode_kernel(DecodeParams p) {
 #endif
 }
 
+constexpr uint32_t kLdsAlone = 80 * 1024;  // half of a CU's LDS; the kernels have some of their own
+
 template <int HD, int RT, int NW>
 hipError_t launch_decode_t(const DecodeParams & p, int n_seq, hipStream_t stream) {
     // x: groups of (split, kv head), 8 per round of XCDs (the last round as it is with p.exact), each group's row tiles on
     // one XCD; y: the sequence (the XCD-mapped grid: kv head g's splits at ids = g mod 8, so the kv heads round up to a
     // multiple of 8)
     const int64_t groups = (int64_t)p.max_split * (p.xcd_heads ? (p.n_head_kv + 7) / 8 * 8 : p.n_head_kv);
+    const uint32_t lds = p.alone && NW == 4 ? kLdsAlone : 0;
     const dim3 grid((uint32_t)(p.exact ? groups : (groups + 7) / 8 * 8 * p.n_rowtiles), (uint32_t)n_seq);
     if constexpr (HD == 128 && RT == 4) {  // one query row per Llama-3-8B-shaped sequence (4 query heads per kv head)
         if (p.kv_nt) {
             if (p.f32)
-                hipLaunchKernelGGL((decode_kernel<HD, RT, true, NW, true>), grid, dim3(NW * kWave), 0, stream, p);
+                hipLaunchKernelGGL((decode_kernel<HD, RT, true, NW, true>), grid, dim3(NW * kWave), lds, stream, p);
             else
-                hipLaunchKernelGGL((decode_kernel<HD, RT, false, NW, true>), grid, dim3(NW * kWave), 0, stream, p);
+                hipLaunchKernelGGL((decode_kernel<HD, RT, false, NW, true>), grid, dim3(NW * kWave), lds, stream, p);
             return hipGetLastError();
         }
     }
     if (p.f32)
-        hipLaunchKernelGGL((decode_kernel<HD, RT, true, NW>), grid, dim3(NW * kWave), 0, stream, p);
+        hipLaunchKernelGGL((decode_kernel<HD, RT, true, NW>), grid, dim3(NW * kWave), lds, stream, p);
     else
-        hipLaunchKernelGGL((decode_kernel<HD, RT, false, NW>), grid, dim3(NW * kWave), 0, stream, p);
+        hipLaunchKernelGGL((decode_kernel<HD, RT, false, NW>), grid, dim3(NW * kWave), lds, stream, p);
     return hipGetLastError();
 }
 

@@ -17,16 +17,14 @@ void operator delete(void * p) noexcept { std::free(p); }
 void operator delete(void * p, size_t) noexcept { std::free(p); }
 
 // The longest first, equal lengths as they come, and nothing taken from the heap; on the XCD-mapped grid only with at most
-// 512 live workgroups.
-static bool order_ok(const std::vector<int32_t> & lens, bool xcd, int64_t chunk) {
-    int64_t live = 0;
-    for (int32_t n : lens) live += 8 * ((n + chunk - 1) / chunk);
+// 512 live workgroups and not with one per CU.
+static bool order_ok(const std::vector<int32_t> & lens, int64_t live, bool xcd, bool alone) {
     std::vector<int> want(lens.size());
     std::iota(want.begin(), want.end(), 0);
-    if (!xcd || live <= 512) std::stable_sort(want.begin(), want.end(), [&](int a, int b) { return lens[a] > lens[b]; });
+    if (!xcd || (live <= 512 && !alone)) std::stable_sort(want.begin(), want.end(), [&](int a, int b) { return lens[a] > lens[b]; });
     int got[mx::kMaxSeqPerLaunch];
     const int before = allocations;
-    decode_order(lens.data(), (int)lens.size(), 8, chunk, xcd, got);
+    decode_order(lens.data(), (int)lens.size(), live, xcd, alone, got);
     return allocations == before && std::equal(want.begin(), want.end(), got);
 }
 
@@ -35,7 +33,7 @@ int main() {
     for (int t = 0; t < 4000; t++) {
         std::vector<int32_t> lens(1 + rng() % mx::kMaxSeqPerLaunch);
         for (int32_t & n : lens) n = 1 + rng() % (t % 2 ? 9000 : 5);
-        if (!order_ok(lens, t % 4 >= 2, 128)) {
+        if (!order_ok(lens, t % 3 ? 512 : 513, t % 4 >= 2, t % 8 >= 4)) {
             std::printf("the order of %zu sequences\n", lens.size());
             return 1;
         }
