@@ -846,7 +846,8 @@ int32_t linear_params(const mx_linear_desc * desc, int32_t count, const uint16_t
     p.plan = mx::LinearPlan{-1, 1, 0, 0};
     if (need) p.plan = forced ? *forced : mx::linear_plan(d.M, d.N, d.K, count, ws_bytes - need);
     if (p.plan.bytes > ws_bytes - need)
-        return fail(MX_ATTN_RESOURCE_EXHAUSTED, "workspace of %zu bytes is smaller than the %zu bytes needed", ws_bytes, need + p.plan.bytes);
+        return fail(MX_ATTN_RESOURCE_EXHAUSTED, "workspace of %zu bytes is smaller than the %zu bytes needed", ws_bytes,
+                    need + p.plan.bytes);
     p.counters = reinterpret_cast<uint32_t *>(static_cast<char *>(workspace) + need);
     p.part = reinterpret_cast<float *>(static_cast<char *>(workspace) + need + mx::linear_counter_bytes(p.plan));
     p.x_stride = d.x_stride;
@@ -1188,8 +1189,10 @@ __attribute__((visibility("default"))) int32_t mx_linear_trace_run(
     const float * const * bias, void * workspace, size_t ws_bytes, mx_attn_stream stream, int32_t i, int32_t parts) {
     if (int32_t rc = check_linear_desc(desc, count)) return rc;
     int32_t shape[5] = {};
-    if (desc->M <= mx::kLinearGemvMaxRows || i < 0 || i >= mx_linear_trace_shape(i, desc->K, shape) || parts < 1 || parts > shape[3])
-        return fail(MX_ATTN_INVALID_ARGUMENT, "tile shape %d does not take M %d, K %d in %d parts", i, desc->M, desc->K, parts);
+    if (desc->M <= mx::kLinearGemvMaxRows || i < 0 || i >= mx_linear_trace_shape(i, desc->K, shape) || parts < 1 ||
+        parts > shape[3])
+        return fail(MX_ATTN_INVALID_ARGUMENT, "tile shape %d does not take M %d, K %d in %d parts", i, desc->M, desc->K,
+                    parts);
     const mx::LinearPlan plan = mx::linear_plan_of(i, parts, desc->M, desc->N, count);
     mx::LinearParams p;
     if (int32_t rc = linear_params(desc, count, W, X, Y, gamma, bias, workspace, ws_bytes, p, &plan)) return rc;

@@ -146,7 +146,8 @@ std::vector<PyObject *> items(PyObject * o) {
     return std::vector<PyObject *>(p, p + n);
 }
 
-mx_attn_desc desc(PyObject * const * heads, int32_t n_q, int64_t q_stride, int64_t kv_stride, int64_t out_stride, PyObject * scale) {
+mx_attn_desc desc(PyObject * const * heads, int32_t n_q, int64_t q_stride, int64_t kv_stride, int64_t out_stride,
+                  PyObject * scale) {
     mx_attn_desc d{};
     d.n_head = int32(heads[0]);
     d.n_head_kv = int32(heads[1]);
@@ -197,10 +198,10 @@ PyObject * decode(PyObject * const * a) {
     int32_t rc;
     {
         Unlocked u;
-        rc = t == at::kFloat ? api.decode_f32(&d, n, c.len.data(), data<float>(q), c.k.data(), c.v.data(), data<float>(out), l, ws.data_ptr(),
-                                              (size_t)ws.numel(), stream())
-                             : api.decode(&d, n, c.len.data(), data<uint16_t>(q), c.k.data(), c.v.data(), data<uint16_t>(out), l, ws.data_ptr(),
-                                          (size_t)ws.numel(), stream());
+        rc = t == at::kFloat ? api.decode_f32(&d, n, c.len.data(), data<float>(q), c.k.data(), c.v.data(), data<float>(out), l,
+                                              ws.data_ptr(), (size_t)ws.numel(), stream())
+                             : api.decode(&d, n, c.len.data(), data<uint16_t>(q), c.k.data(), c.v.data(),
+                                          data<uint16_t>(out), l, ws.data_ptr(), (size_t)ws.numel(), stream());
     }
     return rc ? code(rc) : pair(out, a[10], lse, a[11]);
 }
@@ -225,8 +226,8 @@ PyObject * decode_rope(PyObject * const * a) {
 }
 
 // The chunk's descriptor: n_head, n_head_kv, head_dim at heads; p0, causal, n_kv, scale.
-mx_attn_desc chunk(PyObject * const * heads, const at::Tensor & q, const at::Tensor & k, const at::Tensor & out, PyObject * p0, PyObject * causal,
-                   PyObject * n_kv, PyObject * scale) {
+mx_attn_desc chunk(PyObject * const * heads, const at::Tensor & q, const at::Tensor & k, const at::Tensor & out, PyObject * p0,
+                   PyObject * causal, PyObject * n_kv, PyObject * scale) {
     need(q.size(0) <= INT32_MAX);
     mx_attn_desc d = desc(heads, (int32_t)q.size(0), q.stride(0), k.stride(0), out.stride(0), scale);
     d.p0 = int32(p0);
@@ -253,7 +254,8 @@ PyObject * prefill(PyObject * const * a) {
     return rc ? code(rc) : pair(out, a[10], lse, a[11]);
 }
 
-// qkv, k_cache, v_cache, n_head, n_head_kv, head_dim, rope_mode, rope_base, p0, causal, n_kv, scale, out, lse, want_lse, workspace
+// qkv, k_cache, v_cache, n_head, n_head_kv, head_dim, rope_mode, rope_base, p0, causal, n_kv, scale, out, lse, want_lse,
+// workspace
 PyObject * prefill_rope(PyObject * const * a) {
     const at::Tensor & q = rows(a[0], at::kFloat), & k = rows(a[1], at::kHalf), & v = rows(a[2], at::kHalf);
     need(k.stride(0) == v.stride(0));
@@ -317,13 +319,14 @@ PyObject * linear(PyObject * const * a) {
     d.M = (int32_t)x.size(0);
     d.N = (int32_t)N;
     d.K = (int32_t)K;
-    d.flags = (a[3] != Py_None ? MX_LINEAR_RMS_NORM : 0) | (truth(a[6]) ? MX_LINEAR_ACCUMULATE : 0) | (a[4] != Py_None ? MX_LINEAR_BIAS : 0) |
-              (f16 ? MX_LINEAR_OUT_F16 : 0);
+    d.flags = (a[3] != Py_None ? MX_LINEAR_RMS_NORM : 0) | (truth(a[6]) ? MX_LINEAR_ACCUMULATE : 0) |
+              (a[4] != Py_None ? MX_LINEAR_BIAS : 0) | (f16 ? MX_LINEAR_OUT_F16 : 0);
     d.x_stride = x.stride(0);
     d.y_stride = outs[0].stride(0);
     d.eps = (float)real(a[5]);
     const size_t bytes = api.linear_workspace_bytes(&d, (int32_t)n);
-    const at::Tensor work = bytes ? at::empty({(int64_t)std::max<size_t>(bytes, 256)}, x.options().dtype(at::kByte)) : at::Tensor();
+    const int64_t room = (int64_t)std::max<size_t>(bytes, 256);
+    const at::Tensor work = bytes ? at::empty({room}, x.options().dtype(at::kByte)) : at::Tensor();
     int32_t rc;
     {
         Unlocked u;
@@ -349,7 +352,8 @@ PyObject * self_attention(PyObject * const * a) {
     need(x.is_cuda() && x.dim() == 3 && x.is_contiguous() && (t == at::kFloat || t == at::kHalf || t == at::kBFloat16));
     const int64_t B = x.size(0), N = x.size(1), E = x.size(2) / 3;
     const int32_t heads = int32(a[1]);
-    need(x.size(2) % 3 == 0 && heads >= 1 && E % heads == 0 && E / heads >= 1 && B <= INT32_MAX && N <= INT32_MAX && E <= INT32_MAX);
+    need(x.size(2) % 3 == 0 && heads >= 1 && E % heads == 0 && E / heads >= 1);
+    need(B <= INT32_MAX && N <= INT32_MAX && E <= INT32_MAX);
     mx_self_attn_desc d{};
     d.batch = (int32_t)B;
     d.n_tok = (int32_t)N;
@@ -390,18 +394,22 @@ PyObject * bind(PyObject *, PyObject * args) {
     int version;
     Py_ssize_t size[4];
     unsigned long long p[9];
-    if (!PyArg_ParseTuple(args, "i(nnnn)KKKKKKKKK", &version, size, size + 1, size + 2, size + 3, p, p + 1, p + 2, p + 3, p + 4, p + 5, p + 6, p + 7,
-                          p + 8))
+    if (!PyArg_ParseTuple(args, "i(nnnn)KKKKKKKKK", &version, size, size + 1, size + 2, size + 3, p, p + 1, p + 2, p + 3, p + 4,
+                          p + 5, p + 6, p + 7, p + 8))
         return nullptr;
     const size_t own[4] = {sizeof(mx_attn_desc), sizeof(mx_attn_rope), sizeof(mx_linear_desc), sizeof(mx_self_attn_desc)};
     bool same = version == MX_ATTN_ABI_VERSION;
     for (int i = 0; i < 4; i++) same = same && (size_t)size[i] == own[i];
     if (!same) {
-        PyErr_Format(PyExc_ImportError, "dooms_amd._native was built for version %d of the library, which is %d, or for other descriptors: build "
-                     "both with `python -m dooms_amd.build`", (int)MX_ATTN_ABI_VERSION, version);
+        PyErr_Format(PyExc_ImportError,
+                     "dooms_amd._native was built for version %d of the library, which is %d, or for other descriptors: build "
+                     "both with `python -m dooms_amd.build`",
+                     (int)MX_ATTN_ABI_VERSION, version);
         return nullptr;
     }
-    auto set = [](auto & f, unsigned long long v) { f = reinterpret_cast<std::remove_reference_t<decltype(f)>>((uintptr_t)v); };
+    auto set = [](auto & f, unsigned long long v) {
+        f = reinterpret_cast<std::remove_reference_t<decltype(f)>>((uintptr_t)v);
+    };
     set(api.prefill_ws, p[0]);
     set(api.decode, p[1]);
     set(api.decode_f32, p[2]);
@@ -414,7 +422,8 @@ PyObject * bind(PyObject *, PyObject * args) {
     Py_RETURN_NONE;
 }
 
-#define MX_ENTRY(name, n) {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(entry<name, n>)), METH_FASTCALL, nullptr}
+#define MX_ENTRY(name, n) \
+    {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void *>(entry<name, n>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     MX_ENTRY(decode, 14), MX_ENTRY(decode_rope, 14), MX_ENTRY(prefill, 14), MX_ENTRY(prefill_rope, 16), MX_ENTRY(linear, 8),
     MX_ENTRY(self_attention, 4), {"bind", bind, METH_VARARGS, nullptr}, {nullptr, nullptr, 0, nullptr}};

@@ -44,7 +44,8 @@ template <bool NORM>
 __global__ __launch_bounds__(kThreads) void stage_kernel(LinearParams p) {
     __shared__ float red[kWaves];
     if (p.plan.splits > 1)  // the split GEMM's counters (one per thread of the whole grid; the grid has rows > 8)
-        for (int i = blockIdx.x * kThreads + threadIdx.x; i < p.plan.tiles; i += gridDim.x * kThreads) p.counters[i * kCounterStride] = 0u;
+        for (int i = blockIdx.x * kThreads + threadIdx.x; i < p.plan.tiles; i += gridDim.x * kThreads)
+            p.counters[i * kCounterStride] = 0u;
     const float * row = p.x + (int64_t)blockIdx.x * p.x_stride;
     const int kp = (p.K + 63) / 64 * 64;  // staged rows are zero-padded to a multiple of 64 columns
     half_t * dst = p.xh + (int64_t)blockIdx.x * kp;
@@ -406,7 +407,8 @@ __device__ __forceinline__ void gemm_big_tile(const LinearParams & p) {
 #pragma unroll
     for (int i = 0; i < Loads; i++) {
         const int j = i * kBigWaves + wave, row = gemm_block_row<kBK>(j, lane), chunk = gemm_block_chunk<kBK>(j, lane);
-        off[i] = row < kBM ? gemm_load_offset<uint32_t>(m0, row, p.M, kp, chunk) : gemm_load_offset<uint32_t>(n0, row - kBM, p.N, p.K, chunk);
+        off[i] = row < kBM ? gemm_load_offset<uint32_t>(m0, row, p.M, kp, chunk)
+                           : gemm_load_offset<uint32_t>(n0, row - kBM, p.N, p.K, chunk);
     }
     // HALF: what this lane's weight loads of the last step go back (kBigWaves is even: every block of a wave has its swizzle)
     const uint32_t back = HALF ? gemm_half_back(gemm_block_chunk<kBK>(wave, lane)) : 0;
@@ -517,16 +519,16 @@ __global__ __launch_bounds__(kBigThreads, 1) void gemm_big_kernel(LinearParams p
 template <bool OUT16, bool HALF>
 __global__ __launch_bounds__(kBigThreads, 1) void gemm_w192_kernel(LinearParams p) { gemm_big_tile<OUT16, 192, 96, HALF>(p); }
 
-// ---- M > 8, products with too few 256-row tiles for the chip: BM x BN tiles of 4 waves, K cut into p.plan.splits parts ----
+// ---- M > 8, products with too few 256-row tiles for the chip: BM x BN tiles of 4 waves, K cut into p.plan.splits parts
 // Few rows are bound by the weights' stream from HBM (24 x 4096 x 4096: 33.5 MB, 5.2 us at 6.4 TB/s), which needs every
 // CU loading: with whole K a product of N = 4096 has 32 column tiles for 256 CUs, so the parts of K make up the rest
 // (4 parts of 64-column tiles: 256 workgroups). Each workgroup keeps NBUF - 1 steps of both operands in flight straight
-// into LDS (48 to 96 KB), in whole row slices of 256 (BK = 128) or 128 bytes, so its few steps arrive about together. Row r of a
-// tile lies whole in LDS with its 16-byte chunks permuted by the row (chunk ^ r % 16, or ^ r / 2 % 8 with 128-byte rows): the
-// 16-byte operand reads of 16 rows at one chunk hit 16 distinct 4-bank groups. The weights are MFMA operand A, so that
-// a lane holds 4 consecutive outputs of one row (16-byte stores).
-// HALF: K is an odd multiple of 32, as in gemm_big_tile; the last part's last step is half padding. WIDE: the tile's rows span
-// 4 GiB or more, so the lanes' offsets take 64 bits.
+// into LDS (32 to 100 KB), in whole row slices of 256 (BK = 128) or 128 bytes, so its few steps arrive about together.
+// Row r of a tile lies whole in LDS with its 16-byte chunks permuted by the row (chunk ^ r % 16, or ^ r / 2 % 8 with
+// 128-byte rows): the 16-byte operand reads of 16 rows at one chunk hit 16 distinct 4-bank groups. The weights are MFMA
+// operand A, so that a lane holds 4 consecutive outputs of one row (16-byte stores).
+// HALF: K is an odd multiple of 32, as in gemm_big_tile; the last part's last step is half padding. WIDE: the tile's rows
+// span 4 GiB or more, so the lanes' offsets take 64 bits.
 template <bool OUT16, int BM, int BN, int WM, int BK, int NBUF, bool HALF, bool WIDE>
 __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     constexpr int WN = kWaves / WM;                        // waves along the weight rows
@@ -561,7 +563,8 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
     for (int i = 0; i < LPS; i++) {
         const int j = i * kWaves + wave, jb = j < XB ? j : j - XB;
         const int row = gemm_block_row<BK>(jb, lane), chunk = gemm_block_chunk<BK>(jb, lane);
-        off[i] = j < XB ? gemm_load_offset<Offset>(m0, row, p.M, kp, chunk) : gemm_load_offset<Offset>(n0, row, p.N, p.K, chunk);
+        off[i] = j < XB ? gemm_load_offset<Offset>(m0, row, p.M, kp, chunk)
+                        : gemm_load_offset<Offset>(n0, row, p.N, p.K, chunk);
     }
     auto issue = [&](int step, int buf) __attribute__((always_inline)) {
         const int64_t k0 = (int64_t)(s0 + step) * BK * 2;
@@ -648,7 +651,8 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         if (threadIdx.x == 0)
-            s_last = __hip_atomic_fetch_add(p.counters + (int64_t)tile * kCounterStride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(S - 1);
+            s_last = __hip_atomic_fetch_add(p.counters + (int64_t)tile * kCounterStride, 1u, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(S - 1);
         __syncthreads();
         if (!s_last) return;
         __builtin_amdgcn_s_waitcnt(0);
@@ -666,7 +670,8 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
                     for (int i = 0; i < MI; i++)
 #pragma unroll
                         for (int j = 0; j < NJ; j++)
-                            v[e][i][j] = __builtin_bit_cast(float4_t, load16_dev(prs, (k0 + e) * (int)TF * 4 + fb + (i * NJ + j) * kWave * 16));
+                            v[e][i][j] = __builtin_bit_cast(
+                                float4_t, load16_dev(prs, (k0 + e) * (int)TF * 4 + fb + (i * NJ + j) * kWave * 16));
 #pragma unroll
             for (int e = 0; e < SC; e++)
                 if (k0 + e < S)
@@ -715,7 +720,9 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
                 } else {
 #pragma unroll
                     for (int v = 0; v < 4; v++)
-                        if (n + v < p.N) prev[i][v] = OUT16 ? (float)static_cast<const half_t *>(p.y[mi])[o + v] : static_cast<const float *>(p.y[mi])[o + v];
+                        if (n + v < p.N)
+                            prev[i][v] = OUT16 ? (float)static_cast<const half_t *>(p.y[mi])[o + v]
+                                               : static_cast<const float *>(p.y[mi])[o + v];
                 }
             }
 #pragma unroll
@@ -730,7 +737,8 @@ __device__ __forceinline__ void gemm_split_tile(const LinearParams & p) {
             const int64_t o = (int64_t)m * p.y_stride + n;
             if constexpr (OUT16) {
                 half_t * y = static_cast<half_t *>(p.y[mi]) + o;
-                if (whole) *reinterpret_cast<half4_t *>(y) = half4_t{(half_t)acc[i][j][0], (half_t)acc[i][j][1], (half_t)acc[i][j][2], (half_t)acc[i][j][3]};
+                const float4_t a = acc[i][j];
+                if (whole) *reinterpret_cast<half4_t *>(y) = half4_t{(half_t)a[0], (half_t)a[1], (half_t)a[2], (half_t)a[3]};
                 else
 #pragma unroll
                     for (int v = 0; v < 3; v++)

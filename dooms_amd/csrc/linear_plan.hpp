@@ -57,7 +57,8 @@ inline size_t linear_counter_bytes(const LinearPlan & l) { return l.splits > 1 ?
 // The plan of tile shape cfg with K in the given number of parts.
 inline LinearPlan linear_plan_of(int cfg, int splits, int32_t M, int32_t N, int32_t count) {
     const GemmCfg & c = kGemmCfgs[cfg];
-    LinearPlan l{cfg, splits, (int32_t)((int64_t)count * (((int64_t)N + c.bn - 1) / c.bn) * (((int64_t)M + c.bm - 1) / c.bm)), 0};
+    const int64_t tiles = count * (((int64_t)N + c.bn - 1) / c.bn) * (((int64_t)M + c.bm - 1) / c.bm);
+    LinearPlan l{cfg, splits, (int32_t)tiles, 0};
     if (splits > 1) l.bytes = (size_t)l.tiles * splits * c.bm * c.bn * 4 + linear_counter_bytes(l);
     return l;
 }

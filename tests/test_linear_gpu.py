@@ -123,8 +123,8 @@ def test_gemm_ragged_edges(device):
 
 @pytest.mark.parametrize("M,N,K", [(9, 64, 32), (33, 132, 160), (200, 256, 192), (129, 96, 320)])
 def test_gemm_step_counts(device, M, N, K):
-    """K steps of 64 (the last one half zero-padded when K is an odd multiple of 32), odd and even step counts
-    (the GEMM's main loop runs steps in pairs and finishes an odd count alone), the smallest GEMM row count."""
+    """K steps of 64 (the last one half padding when K is an odd multiple of 32), odd and even step counts, the smallest
+    GEMM row count."""
     run(device, 20 + K, M, N, K, norm=True, bias=True)
 
 
@@ -136,14 +136,15 @@ def test_gemm_few_rows(device, M, N):
 
 @pytest.mark.parametrize("M", [9, 16, 17, 32, 33, 64, 65, 128, 129, 300])
 @pytest.mark.parametrize("N,K,opts", [
-    (136, 2048, dict(bias=True, accumulate=True)),         # K a multiple of 128: every tile shape, K in parts
+    (136, 2048, dict(bias=True, accumulate=True)),         # K a multiple of 128: any tile shape may be taken
     (1029, 1152, dict(norm=True, y_pad=3)),                # the last columns of a row not a whole 16 bytes
     (72, 1056, dict(accumulate=True, out_f16=True)),       # K an odd multiple of 32: the last step half padding
     (200, 640, dict(bias=True, out_f16=True, count=3)),
 ])
 def test_gemm_parts_of_k(device, M, N, K, opts):
-    """Few tiles: K is cut into parts merged by the last of a tile's workgroups; rows at the edges of every tile height,
-    columns that end inside a tile, and outputs written whole and in pieces."""
+    """Few tiles: K is cut into parts merged by the last of a tile's workgroups, on the shapes that the plan takes for
+    these rows (test_linear_shapes_gpu runs every shape and number of parts); columns that end inside a tile, and outputs
+    written whole and in pieces."""
     run(device, 80 + M + K, M, N, K, **opts)
 
 
@@ -193,10 +194,9 @@ def test_gemm_workspace_of_the_staged_rows_alone(device, M, N, K):
         assert np.array_equal(outs[0], outs[1])
 
 
-def test_gemm_big_tiles_ragged(device):
-    """A product with enough 256 x 256 tiles for the large-tile GEMM: M and N not multiples of 256 (rows and
-    columns past them repeat the last one and are never stored), 5 steps of 32 columns, with the RMS normalization,
-    bias and accumulation; rows sampled across the tiles and at both edges."""
+def test_gemm_many_tiles_ragged_norm(device):
+    """Many tiles and a short K: M and N not multiples of a tile (rows and columns past them repeat the last one and are
+    never stored), with the RMS normalization, bias and accumulation; rows sampled across the tiles and at both edges."""
     run(device, 10, 1300, 8300, 160, norm=True, bias=True, accumulate=True,
         rows=[0, 1, 255, 256, 511, 700, 1023, 1024, 1279, 1280, 1299])
 
@@ -211,27 +211,25 @@ def test_gemm_large_tiles_odd_k(device, M, N, K, opts):
     run(device, 15, M, N, K, rows=[0, 1, 255, 256, 1023, 1024, M - 2, M - 1], **opts)
 
 
-def test_gemm_mid_tiles_ragged(device):
-    """Enough 256 x 128 tiles (but too few 256 x 256 ones) for the 256 x 128 GEMM: ragged M and N, 3 steps of 32
-    columns, f16 output with bias."""
+def test_gemm_many_tiles_ragged_f16(device):
+    """The same for an f16 output with bias."""
     run(device, 11, 1900, 3896, 96, bias=True, out_f16=True, rows=[0, 1, 255, 256, 1023, 1536, 1791, 1792, 1899])
 
 
-def test_gemm_w192_tiles_ragged(device):
-    """A product that takes the 256 x 192 tiles (8 waves of 64 x 96 columns, the B tile's 12 load blocks spread over
-    16 loads): ragged M and N, 3 steps of 32 columns, accumulation."""
+def test_gemm_many_tiles_ragged_accumulate(device):
+    """The same accumulating, N not a multiple of 8."""
     run(device, 12, 1900, 5700, 96, accumulate=True, rows=[0, 1, 255, 256, 1023, 1536, 1791, 1792, 1899])
 
 
 @pytest.mark.parametrize("K", [64, 192, 320])
 @pytest.mark.parametrize("M,N,opts", [
-    (1300, 8300, dict(norm=True, bias=True, accumulate=True)),  # 256 x 256 tiles
-    (1900, 3896, dict(bias=True, out_f16=True)),                # 256 x 128 tiles
-    (1900, 5700, dict(accumulate=True)),                        # 256 x 192 tiles
+    (1300, 8300, dict(norm=True, bias=True, accumulate=True)),
+    (1900, 3896, dict(bias=True, out_f16=True)),
+    (1900, 5700, dict(accumulate=True)),
 ])
 def test_gemm_tiles_ragged_k64_steps(device, M, N, opts, K):
-    """The same ragged products with K a multiple of 64, which the tiled GEMMs walk in steps of 64 columns through
-    two LDS buffers: one step, three and five (the buffer ring wrapping at an odd count)."""
+    """The same ragged products with K a multiple of 64: one step of 64 columns, three and five (two LDS buffers wrapping
+    at an odd count)."""
     run(device, 13 + K, M, N, K, rows=[0, 1, 255, 256, 1023, 1024, M - 2, M - 1], **opts)
 
 
