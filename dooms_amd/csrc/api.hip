@@ -140,8 +140,8 @@ DecodeShape decode_shape(const mx_attn_desc * d) {
 //   * sequences of up to 256 keys whole, without a merge, one 32-key block per wave of 8: 8 x 160 keys of 20 kv heads
 //     7.5 -> 6.0 us, 5 x 129 keys of 8 kv heads 6.6 -> 6.1; not f32 rows of head dim 128 with more than 4 rows per kv
 //     head, where the wider tile's merge of 8 waves costs more (256 keys of Qwen2.5-7B 8.2 -> 8.5), nor f32 rows of head
-//     dim 64 past one workgroup per CU, which is what their registers allow (12 x 130 keys of 20 kv heads 7.0 split,
-//     8.1 whole; f16 rows fit two and stay ahead: 16 x 140 keys 7.6 -> 6.4), nor where the workgroup cap leaves the
+//     dim 64 past one workgroup per CU, which is what their registers allow (12 x 130 keys of 32 kv heads 7.8 split,
+//     10.2 whole; f16 rows fit two and stay ahead: 16 x 140 keys 7.6 -> 6.4), nor where the workgroup cap leaves the
 //     sequences whole anyway, on 4 waves (32 x 140 keys of 28 kv heads, f16, 10.6 on 4 waves, 12.1 on 8);
 //   * head dim 64, several sequences: at most 16 splits, the most that one round of the merge folds, with twice the
 //     waves per split (3 x 3096 keys of 2 kv heads 10.8 -> 10.1). On f32 rows a CU holds one such workgroup: where the
@@ -219,16 +219,14 @@ bool decode_alone(bool f32, int head_dim, int waves, int64_t live, bool xcd) {
 }
 
 // The order of a launch's sequences in its grid: the longest first, so that the workgroups past a shorter one's splits come
-// late (f16 rows in random order, us: 16 Llama-3-8B caches of 87-700 keys 13.3 -> 11.7, 16 Qwen2.5-7B caches of 1.3k-7.3k
-// 35.5 -> 33.1). On the XCD-mapped grid not with more live workgroups than run at once (two per CU: later ones fill the
-// gaps there, and the sorted order ran up to 3 % slower, 16 Llama-3-8B caches of 325-2600 keys 26.7 against 27.5), nor with
-// one per CU (decode_alone: level on average, at worst 1.04x). Equal lengths keep the caller's order. By insertion:
-// std::stable_sort takes a buffer from the heap, and a decode call must not.
-void decode_order(const int32_t * kv_len, int n_seq, int64_t live, bool xcd, bool alone, int * order) {
-    const bool sort = !xcd || (live <= 512 && !alone);
+// late (f16 rows in random order: 16 Qwen2.5-7B caches of 1.3k-7.3k 35.5 -> 33.1 us). Not on the XCD-mapped grid: its
+// launches gain 1 % on average, but up to 1.39x is lost near a full round of the CUs (3 caches of up to 6980 keys, 64 heads
+// over 8 kv heads, fused step, 14.1 us against 18.9; 12 of up to 1182, Llama-3-8B, f16, 10.8 against 12.5). Equal lengths
+// keep the caller's order. By insertion: std::stable_sort takes a buffer from the heap, and a decode call must not.
+void decode_order(const int32_t * kv_len, int n_seq, bool xcd, int * order) {
     for (int i = 0; i < n_seq; i++) {
         int at = i;
-        for (; sort && at > 0 && kv_len[order[at - 1]] < kv_len[i]; at--) order[at] = order[at - 1];
+        for (; !xcd && at > 0 && kv_len[order[at - 1]] < kv_len[i]; at--) order[at] = order[at - 1];
         order[at] = i;
     }
 }
@@ -638,7 +636,7 @@ int32_t decode_impl(const mx_attn_desc * desc, int32_t batch, const int32_t * kv
         for (int i = 0; i < n_seq; i++) live += (kv_len[b0 + i] + chunk - 1) / chunk * d.n_head_kv * s.n_rowtiles;
         p.alone = decode_alone(f32, d.head_dim, plan.waves, live, p.xcd_heads);
         int order[mx::kMaxSeqPerLaunch];
-        decode_order(kv_len + b0, n_seq, live, p.xcd_heads, p.alone, order);
+        decode_order(kv_len + b0, n_seq, p.xcd_heads, order);
         p.max_split = 1;
         int32_t groups = 0;
         for (int i = 0; i < n_seq; i++) {

@@ -16,15 +16,14 @@ void * operator new(size_t n, const std::nothrow_t &) noexcept { return operator
 void operator delete(void * p) noexcept { std::free(p); }
 void operator delete(void * p, size_t) noexcept { std::free(p); }
 
-// The longest first, equal lengths as they come, and nothing taken from the heap; on the XCD-mapped grid only with at most
-// 512 live workgroups and not with one per CU.
-static bool order_ok(const std::vector<int32_t> & lens, int64_t live, bool xcd, bool alone) {
+// The longest first, equal lengths as they come, and nothing taken from the heap; on the XCD-mapped grid as they come.
+static bool order_ok(const std::vector<int32_t> & lens, bool xcd) {
     std::vector<int> want(lens.size());
     std::iota(want.begin(), want.end(), 0);
-    if (!xcd || (live <= 512 && !alone)) std::stable_sort(want.begin(), want.end(), [&](int a, int b) { return lens[a] > lens[b]; });
+    if (!xcd) std::stable_sort(want.begin(), want.end(), [&](int a, int b) { return lens[a] > lens[b]; });
     int got[mx::kMaxSeqPerLaunch];
     const int before = allocations;
-    decode_order(lens.data(), (int)lens.size(), live, xcd, alone, got);
+    decode_order(lens.data(), (int)lens.size(), xcd, got);
     return allocations == before && std::equal(want.begin(), want.end(), got);
 }
 
@@ -33,7 +32,7 @@ int main() {
     for (int t = 0; t < 4000; t++) {
         std::vector<int32_t> lens(1 + rng() % mx::kMaxSeqPerLaunch);
         for (int32_t & n : lens) n = 1 + rng() % (t % 2 ? 9000 : 5);
-        if (!order_ok(lens, t % 3 ? 512 : 513, t % 4 >= 2, t % 8 >= 4)) {
+        if (!order_ok(lens, t % 4 >= 2)) {
             std::printf("the order of %zu sequences\n", lens.size());
             return 1;
         }
