@@ -44,7 +44,7 @@ struct DecodeParams {
     int32_t xcd_heads;   // 1: kv head g's splits run on XCD g % 8 (n_head_kv a multiple of 8, or one short sequence)
     int32_t exact;       // 1: no padding in the grid: every sequence has max_split splits (one row tile, no xcd_heads)
     int32_t alone;       // 1: the launch asks for LDS enough that a CU holds one workgroup (4 waves)
-    int32_t kv_nt;       // 1: non-temporal K/V loads (one long sequence with xcd_heads, or at least 256 MB of K/V);
+    int32_t kv_nt;       // 1: non-temporal K/V loads (at least 16 MB of K/V with xcd_heads, or at least 256 MB);
                          // honoured by the head-dim-128 kernels with 4-row tiles
     float scale_log2;    // scale * log2(e): scores are kept in base-2 units
     int32_t f32;         // 1: f32 query rows in qkv (q_stride floats apart) and f32 output in out32

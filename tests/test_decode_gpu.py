@@ -419,3 +419,19 @@ def test_equal_splits(device, H, G, hd, lens, f32):
     for b, n in enumerate(lens):
         ro, rl = ref_attention(q[b:b + 1].numpy(), *caches[b], H, G, hd, 1.0 / np.sqrt(hd), p0=n - 1, causal=False)
         assert_close(out[b:b + 1].cpu().numpy().astype(np.float64), ro, hd, f"sequence {b} of {n} keys", lse[b:b + 1].cpu().numpy(), rl)
+
+
+# ragged f32 launches of head dim 128 either side of the workgroups up to which a CU holds one (223 on the XCD-mapped grid, 191
+# off it), on each row tile
+@pytest.mark.parametrize("H,G,splits", [(32, 8, 27), (32, 8, 28), (64, 8, 27), (96, 8, 28), (28, 4, 47), (28, 4, 48), (5, 5, 38), (48, 3, 64)])
+def test_one_workgroup_per_cu(device, H, G, splits):
+    lens = [128 * n - 3 for n in (splits // 2, splits // 3)]
+    lens.append(128 * (splits - splits // 2 - splits // 3) - 100)
+    rng = np.random.default_rng(H + splits)
+    q = torch.from_numpy(normal_f16(rng, (3, H * 128), 1.0))
+    caches = [[normal_f16(rng, (n, G * 128), 1.0) for _ in range(2)] for n in lens]
+    ks, vs = ([torch.from_numpy(c[i]).to(device) for c in caches] for i in range(2))
+    out, lse = A.decode(q.to(device, torch.float32), ks, vs, lens, n_head=H, n_head_kv=G, head_dim=128, want_lse=True)
+    for b, n in enumerate(lens):
+        ro, rl = ref_attention(q[b:b + 1].numpy(), *caches[b], H, G, 128, 1.0 / np.sqrt(128), p0=n - 1, causal=False)
+        assert_close(out[b:b + 1].cpu().numpy().astype(np.float64), ro, 128, f"sequence {b} of {n} keys", lse[b:b + 1].cpu().numpy(), rl)
